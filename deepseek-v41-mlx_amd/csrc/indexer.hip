@@ -553,8 +553,8 @@ __global__ __launch_bounds__(kMxThreads) void indexer_score_mx_kernel(
   }
 }
 
-// Prefill (many queries per batch row, no candidate mask): a workgroup scores 8 consecutive
-// queries of one batch row -- one per wave -- against a range of kPfRows keys. The keys stream
+// Prefill (many queries per batch row): a workgroup scores 8 consecutive queries of one batch row
+// -- one per wave -- against a range of at most kPfRows keys. The keys stream
 // through an LDS ring in 64-row chunks with global_load_lds, so each key row is read from HBM
 // once per workgroup instead of once per query; a wave holds its query's [heads x 128] block
 // as MFMA A operands in registers and reads every chunk's B operands from LDS. Rows are stored
@@ -562,23 +562,38 @@ __global__ __launch_bounds__(kMxThreads) void indexer_score_mx_kernel(
 // touches fall in distinct banks. Per chunk a wave runs 4 tiles x 4 k-steps x HT head tiles of
 // 16x16x32 MFMA and the same epilogue as the decode kernel; queries mask rows past their own
 // causal length, rows past the group's longest one are written as -inf without compute.
+//
+// CAND: with a candidate mask (index sources below the candidate source, indexer.py:131-132). Each
+// wave packs its query's mask bytes of the range into bits in LDS once, before the key loop; a
+// 16-row tile none of whose rows is a visible candidate of the query is not multiplied. Masked
+// chunks used to run on the decode kernel, one workgroup per query and row range, which reads every
+// key again for every query: 2,048 queries x 32,768 keys, 32 heads, half of the entries kept,
+// 1,181 us there with the selection fused against 387 us here (+ 297 us for the selection).
 constexpr int kPfThreads = 512;        // 8 waves = 8 queries
 constexpr int kPfChunk = 64;           // key rows per ring slot (16 KB at 128 channels)
 constexpr int kPfSlots = 3;            // ring slots: 2 chunks in flight (48 KB: two workgroups per CU)
-constexpr int kPfRows = 2048;          // key rows per workgroup
+constexpr int kPfRows = 2048;          // most key rows per workgroup
+
+// One bit per byte of v: bit i set where byte i is not 0.
+__device__ __forceinline__ uint32_t nonzero_bytes(uint32_t v) {
+  const uint32_t t = (v | ((v & 0x7F7F7F7Fu) + 0x7F7F7F7Fu)) & 0x80808080u;   // bit 7 of each non-zero byte
+  return ((t >> 7) * 0x10204080u) >> 28;   // bits 0, 8, 16, 24 -> 28, 29, 30, 31 (no two products overlap)
+}
 
 // (__launch_bounds__'s second argument, 4 waves per SIMD, caps VGPRs at 128 so that two
 // workgroups share a CU)
-template <int HT>
+template <int HT, bool CAND>
 __global__ __launch_bounds__(kPfThreads, 4) void indexer_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ w_raw, float w_scale, const bf16_t* __restrict__ kcache,
-    int64_t k_bstride, float* __restrict__ scores, int n, int nb, int start_pos, int ratio) {
+    int64_t k_bstride, const uint8_t* __restrict__ cand, float* __restrict__ scores, int n, int nb, int start_pos,
+    int ratio, int rows_per_wg, int cand_vec) {
   constexpr int H = HT * 16, DIM = 128, KS = 4;
   constexpr int ROWB = DIM * 2;                          // 256 bytes per key row
   constexpr int CHUNKB = kPfChunk * ROWB;
   constexpr int NL = CHUNKB / 1024 / (kPfThreads / 64);  // copies per wave per chunk
   static_assert(NL * 1024 * (kPfThreads / 64) == CHUNKB, "a chunk splits evenly into 1 KB copies per wave");
   __shared__ __align__(16) uint8_t ring[kPfSlots * CHUNKB];
+  __shared__ __align__(8) uint32_t cbits[CAND ? kPfThreads / 64 : 1][CAND ? kPfRows / 32 : 2];
 
   const int groups = (n + 7) / 8;
   const int b = blockIdx.y / groups, sg = blockIdx.y - (blockIdx.y / groups) * groups;
@@ -589,7 +604,7 @@ __global__ __launch_bounds__(kPfThreads, 4) void indexer_prefill_kernel(
   const int s_last = min(sg * 8 + 7, n - 1);
   const int lens_max = (start_pos + s_last + 1) / ratio;
   const int lens = (start_pos + min(s, n - 1) + 1) / ratio;
-  const int r0 = blockIdx.x * kPfRows, r1 = min(r0 + kPfRows, nb);
+  const int r0 = blockIdx.x * rows_per_wg, r1 = min(r0 + rows_per_wg, nb);
   const int vis_end = max(r0, min(r1, lens_max));
   float* out = scores + ((int64_t)b * n + min(s, n - 1)) * nb;
   // rows past the group's visibility: -inf for each of its queries
@@ -635,6 +650,31 @@ __global__ __launch_bounds__(kPfThreads, 4) void indexer_prefill_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) wv[ht][i] = round_bf16(bf2f(wrow[ht * 16 + 4 * g + i]) * w_scale);
   }
+  if constexpr (CAND) {                    // this wave's mask bits: lane l holds rows r0 + 32 l .. + 31
+    const uint8_t* cr = cand + qi * nb + r0;
+    const int left = min(r1, lens) - r0;   // bytes past the range or the query's visibility stay 0
+    uint32_t bits = 0u;
+    if (cand_vec) {                        // rows of the mask 16-byte aligned (nb a multiple of 16)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        if (32 * lane + 16 * h < left) {
+          const uint4 m = *reinterpret_cast<const uint4*>(cr + 32 * lane + 16 * h);
+          bits |= (nonzero_bytes(m.x) | nonzero_bytes(m.y) << 4 | nonzero_bytes(m.z) << 8 | nonzero_bytes(m.w) << 12)
+                  << (16 * h);
+        }
+      }
+      const int keep = left - 32 * lane;   // the last piece may reach past the query's visibility
+      if (keep < 32) bits &= keep > 0 ? (1u << keep) - 1u : 0u;
+    } else {                               // 64 bytes per load, packed by a ballot
+#pragma unroll 8
+      for (int j = 0; j < kPfRows / 64; ++j) {
+        const int t = 64 * j + lane;
+        const uint64_t m = __ballot(t < left && cr[min(t, max(left - 1, 0))] != 0);
+        bits = lane == 2 * j ? (uint32_t)m : (lane == 2 * j + 1 ? (uint32_t)(m >> 32) : bits);
+      }
+    }
+    cbits[wave][lane] = bits;              // read back by this wave only
+  }
   // query, weights and chunk 0 complete (a wait the compiler sees: no drain inside the loop)
   __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
   for (int c = 1; c < nchunks && c < kPfSlots - 1; ++c) issue(c);
@@ -648,8 +688,19 @@ __global__ __launch_bounds__(kPfThreads, 4) void indexer_prefill_kernel(
     __syncthreads();                       // chunk c landed for every wave; chunk c-1 consumed
     if (c + kPfSlots - 1 < nchunks) issue(c + kPfSlots - 1);
     const uint8_t* buf = ring + (c % kPfSlots) * CHUNKB;
+    float part[4];                         // this lane's head group's share of the chunk's four 16-row tiles
+    static_assert(kPfChunk == 64, "four 16-row tiles per chunk, one row per lane");
+    uint32_t mlo = 0u, mhi = 0u;           // the chunk's mask bits (CAND)
+    if constexpr (CAND) {
+      const uint2 m = *reinterpret_cast<const uint2*>(&cbits[wave][2 * c]);
+      mlo = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.x);
+      mhi = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.y);
+    }
 #pragma unroll
-    for (int kt = 0; kt < kPfChunk / 16; ++kt) {
+    for (int kt = 0; kt < 4; ++kt) {
+      part[kt] = 0.0f;
+      if constexpr (CAND)                  // wave-uniform
+        if ((((kt < 2 ? mlo : mhi) >> (16 * (kt & 1))) & 0xFFFFu) == 0u) continue;
       f32x4 acc[HT];
 #pragma unroll
       for (int ht = 0; ht < HT; ++ht) acc[ht] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -660,16 +711,29 @@ __global__ __launch_bounds__(kPfThreads, 4) void indexer_prefill_kernel(
 #pragma unroll
         for (int ht = 0; ht < HT; ++ht) acc[ht] = mfma16x16x32(qa[ht][ks], kop, acc[ht]);
       }
-      float part = 0.0f;
 #pragma unroll
       for (int ht = 0; ht < HT; ++ht)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) part += relu_bits(acc[ht][i]) * wv[ht][i];
-      part = sum_rows4(part);
-      const int row = r0 + c * kPfChunk + kt * 16 + l16;
-      if (qok && g == 0 && row < vis_end) out[row] = row < lens ? part : -INFINITY;
+        for (int i = 0; i < 4; ++i) part[kt] += relu_bits(acc[ht][i]) * wv[ht][i];
     }
+    // lane = row of the chunk (row group g holds tile g's sums): one 256-byte store per wave. Summing
+    // and storing tile by tile (8 permutes and 8 additions more, four 64-byte stores): 8,192 queries x
+    // 10,240 keys x 64 heads 945 us, 911 us this way, in turn.
+    const float v = sum_rows4x4(part[0], part[1], part[2], part[3]);
+    const int row = r0 + c * kPfChunk + lane;
+    bool seen = row < lens;
+    if constexpr (CAND) seen = (((lane < 32 ? mlo : mhi) >> (lane & 31)) & 1u) != 0u;
+    if (qok && row < vis_end) out[row] = seen ? v : -INFINITY;
   }
+}
+
+// Key rows per prefill workgroup: kPfRows, halved down to 256 while fewer than 512 workgroups (two
+// per CU) would run: a chunk of a few dozen queries leaves most of the chip idle otherwise (64 heads,
+// 10,240 keys: 8 queries 54.5 -> 12.5 us, 64 queries 55.9 -> 19.2 us, 512 queries 98.9 -> 80.3 us).
+static int prefill_rows(int64_t groups, int nb) {
+  int r = kPfRows;
+  while (r > 256 && groups * ((nb + r - 1) / r) < 512) r /= 2;
+  return r;
 }
 
 // fp32 path (parity configs): one thread per cache row, the query's q and w in LDS.
@@ -759,19 +823,21 @@ extern "C" int dsv41_indexer_score(const void* q, const void* w_raw, float w_sca
   if (dtype != DSV41_BF16) return set_error(DSV41_E_DTYPE, "%s: dtype %d not supported", what, dtype);
   DSV41_REQUIRE(aligned16(q) && aligned16(index_k), DSV41_E_ARG, "%s: q and index_k must be 16-byte aligned", what);
   DSV41_REQUIRE(k_bstride % 8 == 0, DSV41_E_ARG, "%s: k_bstride must be a multiple of 8", what);
-  if (n >= 8 && !candidates && dim == 128 && (heads == 64 || heads == 32 || heads == 16) &&
+  if (n >= 8 && dim == 128 && (heads == 64 || heads == 32 || heads == 16) &&
       (int64_t)bsz * ((n + 7) / 8) < 65536) {
-    const dim3 pgrid((unsigned)((nb + kPfRows - 1) / kPfRows), (unsigned)(bsz * ((n + 7) / 8)));
-#define DSV41_PF_CASE(HT_)                                                                                  \
-    if (heads == HT_ * 16) {                                                                                 \
-      hipLaunchKernelGGL((indexer_prefill_kernel<HT_>), pgrid, dim3(kPfThreads), 0, stream, (const bf16_t*)q, \
-                         (const bf16_t*)w_raw, w_scale, (const bf16_t*)index_k, k_bstride, scores, n, nb,      \
-                         start_pos, ratio);                                                                  \
+    const int64_t groups = (int64_t)bsz * ((n + 7) / 8);
+    const int rows = prefill_rows(groups, nb);
+    const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
+    const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
+#define DSV41_PF_CASE(HT_, CAND_)                                                                           \
+    if (heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                             \
+      hipLaunchKernelGGL((indexer_prefill_kernel<HT_, CAND_>), pgrid, dim3(kPfThreads), 0, stream,           \
+                         (const bf16_t*)q, (const bf16_t*)w_raw, w_scale, (const bf16_t*)index_k, k_bstride,   \
+                         candidates, scores, n, nb, start_pos, ratio, rows, cvec);                           \
       return check_launch(what);                                                                             \
     }
-    DSV41_PF_CASE(4)
-    DSV41_PF_CASE(2)
-    DSV41_PF_CASE(1)
+    DSV41_PF_CASE(4, false) DSV41_PF_CASE(2, false) DSV41_PF_CASE(1, false)
+    DSV41_PF_CASE(4, true) DSV41_PF_CASE(2, true) DSV41_PF_CASE(1, true)
 #undef DSV41_PF_CASE
   }
   int rows_per_wg = 0;

@@ -89,6 +89,19 @@ __device__ __forceinline__ float sum_rows4(float v) {
   return __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
 }
 
+// sum_rows4 of four values at once: lane (row g, l) of the result holds the sum of the g-th value
+// over the four 16-lane rows, with sum_rows4's additions ((r0 + r1) + (r2 + r3)), in 3 permutes and
+// 3 additions instead of 8 and 8. permlane16_swap(a, b) gives rows (a0, b0, a2, b2) and
+// (a1, b1, a3, b3); permlane32_swap(c, d) gives (c0, c1, d0, d1) and (c2, c3, d2, d3).
+__device__ __forceinline__ float sum_rows4x4(float v0, float v1, float v2, float v3) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v0), __float_as_uint(v1), false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v2), __float_as_uint(v3), false, false);
+  const float c = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const float d = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  const auto e = __builtin_amdgcn_permlane32_swap(__float_as_uint(c), __float_as_uint(d), false, false);
+  return __uint_as_float(e[0]) + __uint_as_float(e[1]);
+}
+
 // max(x, 0) as one integer max of the bits: a negative float has the sign bit set, so it becomes
 // +0.0, and a non-negative one passes unchanged. fmaxf(x, 0.0f) costs two v_max_f32 in IEEE mode
 // (the first quiets a signalling NaN); this differs from it only for NaN inputs and in giving +0.0

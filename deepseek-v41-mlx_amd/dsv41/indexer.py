@@ -42,6 +42,15 @@ def select_candidate_blocks(scores: torch.Tensor, lens, topk_blocks: int,
                                  _lens_tensor(lens, scores.device))
 
 
+# Queries per sequence from which bf16 keys take the scoring and the selection as two calls: the
+# scoring kernel then reads each key once per 8 queries, where the fused form's reads every key for
+# every query. Only masked layers meet the choice (without a mask the fused form stops at 8 queries
+# anyway). 32 heads, fused against score + select: 8 queries x 65,536 keys 42.9 against 30.1 us,
+# 64 x 8,192 22.0 against 21.7 us, 2,048 x 32,768 1,181 against 684 us; no size measured from 8
+# queries on favoured the fused form.
+CHUNK_QUERIES = 8
+
+
 def weight_scale(n_heads: int, head_dim: int, dtype) -> float:
     """head_dim**-0.5 * n_heads**-0.5 as the activation dtype holds it: a python scalar
     multiplying an MLX array takes the array's dtype (indexer.py:123)."""
@@ -151,7 +160,7 @@ class Indexer(torch.nn.Module):
                 q = _abi.rope_tail(q, rd, cos, sin, start_pos, 1)
             else:
                 _abi.index_q_prep(q, cos, sin, rd, start_pos)
-            if not self.is_candidate_source and q.dtype == torch.bfloat16:
+            if not self.is_candidate_source and q.dtype == torch.bfloat16 and n < CHUNK_QUERIES:
                 # decode shapes the fused form serves: the same selection, the scores never written
                 idx = _abi.indexer_topk(q, w_raw, w_scale, index_k, start_pos, self.ratio, self.index_topk, offset,
                                         cand)

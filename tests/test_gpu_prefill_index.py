@@ -1,0 +1,70 @@
+"""The chunk (8 or more queries) forms of the indexer against the one-query kernels: the same scores, bit for bit."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(b, n, heads, nb, seed, spare=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    q = torch.randn(b, n, heads, 128, generator=g, device="cuda").bfloat16()
+    w = torch.randn(b, n, heads, generator=g, device="cuda").bfloat16()
+    k = torch.randn(b, nb + spare, 128, generator=g, device="cuda").bfloat16()
+    return g, q, w, k
+
+
+def _per_query(q, w, keys, start, ratio, cand):
+    """Scores of each query by a call of its own (the one-query kernel, a workgroup per query)."""
+    from dsv41 import _abi
+    rows = []
+    for s in range(q.shape[1]):
+        c = None if cand is None else cand[:, s:s + 1].contiguous()
+        rows.append(_abi.indexer_score(q[:, s:s + 1].contiguous(), w[:, s:s + 1].contiguous(), 0.07, keys, start + s,
+                                       ratio, c))
+    return torch.cat(rows, 1)
+
+
+@pytest.mark.parametrize("b,n,heads,nb,start,ratio,keep", [
+    (1, 8, 32, 1, 0, 1, 0.5),            # one key; most queries see it only
+    (2, 9, 64, 63, 40, 1, 0.5),          # partial query group, partial chunk, causal edge inside the range
+    (1, 15, 16, 64, 60, 1, 0.0),         # nothing kept
+    (1, 17, 32, 2047, 8171, 4, 0.05),    # most 16-row tiles empty; odd nb: byte loads of the mask
+    (2, 8, 64, 2048, 8184, 4, 0.5),      # one whole range, vector loads of the mask
+    (1, 24, 32, 2064, 2040, 1, 1.0),     # everything kept; the last range holds 16 rows
+    (1, 16, 32, 4101, 16400, 4, 0.3),    # several ranges, queries before and after the last key
+])
+def test_masked_chunk_scores_equal_per_query(gpu, b, n, heads, nb, start, ratio, keep):
+    from dsv41 import _abi
+    g, q, w, k = _inputs(b, n, heads, nb, nb + n, spare=3)
+    keys = k[:, :nb]                     # a view of a longer cache
+    cand = torch.rand(b, n, (nb + 7) // 8, generator=g, device="cuda").lt(keep).repeat_interleave(8, -1)[..., :nb]
+    cand = cand.to(torch.uint8).mul_(255).contiguous()       # any non-zero byte keeps an entry
+    got = _abi.indexer_score(q, w, 0.07, keys, start, ratio, cand)
+    assert torch.equal(got, _per_query(q, w, keys, start, ratio, cand))
+    assert torch.equal(_abi.indexer_score(q, w, 0.07, keys, start, ratio), _per_query(q, w, keys, start, ratio, None))
+
+
+def test_masked_chunk_unaligned_mask(gpu):
+    """A mask whose rows are whole 16-byte pieces but whose base is not aligned takes the byte loads."""
+    from dsv41 import _abi
+    g, q, w, k = _inputs(1, 10, 32, 256, 5)
+    room = torch.zeros(10 * 256 + 3, dtype=torch.uint8, device="cuda")
+    cand = room[3:].view(1, 10, 256)
+    cand.copy_(torch.rand(1, 10, 256, generator=g, device="cuda").lt(0.2))
+    got = _abi.indexer_score(q, w, 0.07, k, 300, 1, cand)
+    assert torch.equal(got, _abi.indexer_score(q, w, 0.07, k, 300, 1, cand.clone()))
+
+
+@pytest.mark.parametrize("n,nb", [(8, 16385), (64, 8192)])
+def test_masked_selection_same_in_both_forms(gpu, n, nb):
+    """Score + select, the form chunks take, against the fused form where that one serves the shape."""
+    from dsv41 import _abi
+    g, q, w, k = _inputs(1, n, 32, nb, 11)
+    cand = torch.rand(1, n, (nb + 7) // 8, generator=g, device="cuda").lt(0.4).repeat_interleave(8, -1)[..., :nb]
+    cand = cand.contiguous()
+    two = _abi.topk_select(_abi.indexer_score(q, w, 0.07, k, nb - n, 1, cand), 128, nb - n, 1, 7)
+    fused = _abi.indexer_topk(q, w, 0.07, k, nb - n, 1, 128, 7, cand)
+    assert fused is not None and torch.equal(two, fused)
