@@ -5,7 +5,8 @@
 // to mx.argpartition, tests/test_parity.py:17-21), -0.0 equal to +0.0. Output positions are
 // ascending, mapped to idx + offset when idx < lens and -1 otherwise.
 //
-// One 1024-thread workgroup per score row. Rows of up to 32K scores (topk_reg_kernel) keep
+// Many rows (a prompt chunk): topk_stripe_kernel, a workgroup sized to the row's length. Few rows
+// (decode): one 1024-thread workgroup per score row. Rows of up to 32K scores (topk_reg_kernel) keep
 // their keys in registers, J consecutive positions per thread, as order-preserving 32-bit keys;
 // an MSD radix select over digits of 11, 11 and 10 bits finds the k-th best key T and how many
 // T-valued keys to take, then one block scan of per-thread (greater, equal) counts gives each
@@ -229,6 +230,206 @@ __global__ __launch_bounds__(kSelThreads) void topk_merge_kernel(const uint32_t*
   });
 }
 
+// Many rows (a prompt chunk's queries): one workgroup of NT threads per row, wave w holding the
+// contiguous positions 64 J w .. + 64 J - 1 of the row in registers, 64 at a time (entry j of lane l:
+// 64 (J w + j) + l). Against topk_reg_kernel's J consecutive positions per thread, the loads and the
+// output are contiguous over the lanes, ranks come from ballots (two instructions per 64 entries
+// instead of a loop over each thread's own), and a barrier holds 4 or 8 waves instead of 16 while the
+// CU's other rows go on. Bound by issue: the per-entry code is straight-line vector code -- an entry
+// that a pass does not count adds to a dummy word of its lane's bank instead of being branched
+// around, and the scalar unit, which the CU's waves share, is left to the output step (with exec
+// masks and uniform branches per entry the same kernel took 267 us at 8,192 rows x 10,240, 408 us at
+// 8,192 x 16,384; topk_reg_kernel 238 and 271 us; this one 84.5 and 128.5 us, 4.8 and 4.3 TB/s of
+// scores and positions).
+//
+// Entries past the row's end have key 0, below every real key but the all-ones NaN's, whose
+// entries all precede them: they are never taken (k < nb: there are enough real entries).
+template <int NT>
+struct StripeShared {
+  uint32_t hist[2][2048 + 64];   // the last 64 words: what a pass does not count
+  uint32_t wsum[NT / 64];
+  uint32_t pick[3];
+};
+
+// LISTS: stage 1 of the two-stage selection (below) over `chunks` chunks of `chunk` entries per row:
+// workgroup (row, chunk) writes its chunk's best min(k, count) as (order key, position).
+template <int NT, int J, bool LISTS>
+__global__ __launch_bounds__(NT, 8) void topk_stripe_kernel(
+    const float* __restrict__ scores, int32_t* __restrict__ out, int n, int row_len, int k_max, int start_pos,
+    int ratio, int offset, int chunks, int chunk, uint32_t* __restrict__ ckey, int32_t* __restrict__ cpos) {
+  constexpr int NBIN = 2048, NW = NT / 64, BPT = NBIN / NT;
+  static_assert(BPT % 2 == 0, "a thread's bins are read 8 bytes at a time");
+  __shared__ __align__(16) StripeShared<NT> sh;
+  const uint32_t row = LISTS ? blockIdx.x / (unsigned)chunks : blockIdx.x;
+  const int ch = LISTS ? (int)(blockIdx.x - row * (unsigned)chunks) : 0;
+  const int nb = LISTS ? min(chunk, row_len - ch * chunk) : row_len;   // entries of this selection
+  const int k = LISTS ? min(k_max, nb) : k_max;
+  const char* x = reinterpret_cast<const char*>(scores + (int64_t)row * row_len + ch * chunk);
+  char* o = reinterpret_cast<char*>(out + (int64_t)row * k);
+  const int64_t list = (int64_t)blockIdx.x * k_max;   // this chunk's list (LISTS)
+  const int s = (int)(row % (unsigned)n);   // 32 bits: the 64-bit division is a long scalar routine
+  const int lens = (start_pos + s + 1) / ratio;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if constexpr (LISTS) {
+    if (k == nb) {                                 // a last chunk of at most k entries goes whole (uniform)
+      for (int t = tid; t < nb; t += NT) {
+        ckey[list + t] = order_key(reinterpret_cast<const float*>(x)[t]);
+        cpos[list + t] = ch * chunk + t;
+      }
+      return;
+    }
+  }
+  int p0 = wave * (64 * J) + lane;                 // this lane's first position
+  // The positions p0 + 64 j are formed again where they are used: kept, they would take J registers.
+  auto forget = [&]() { asm volatile("" : "+v"(p0)); };
+  uint32_t key[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    key[j] = __float_as_uint(*reinterpret_cast<const float*>(x + (uint32_t)min(p0 + 64 * j, nb - 1) * 4u));
+    if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);     // no more than 4 entries' temporaries at once
+  }
+  auto clear = [&](int b) {
+    uint2* h = reinterpret_cast<uint2*>(sh.hist[b]);
+#pragma unroll
+    for (int i = 0; i < NBIN / 2 / NT; ++i) h[tid + i * NT] = make_uint2(0u, 0u);
+  };
+  clear(0);
+  clear(1);
+  forget();
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    key[j] = p0 + 64 * j < nb ? order_key(__uint_as_float(key[j])) : 0u;
+    if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+  }
+  __syncthreads();
+
+  uint32_t prefix = 0u;                            // resolved top bits of the k-th best key, in place
+  int need = k;                                    // entries still to take from the prefix's bin
+  bool whole = false;                              // the bin holds exactly `need` entries
+#pragma unroll
+  for (int pass = 0; pass < 3; ++pass) {
+    const int shift = pass == 0 ? 21 : (pass == 1 ? 10 : 0);
+    uint32_t* h = sh.hist[pass & 1];
+    const uint32_t dummy = NBIN + lane;
+    forget();
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      uint32_t bin;
+      bool counts;
+      if (pass == 0) {
+        bin = key[j] >> 21;
+        counts = p0 + 64 * j < nb;
+      } else if (pass == 1) {
+        bin = (key[j] >> 10) & 2047u;
+        counts = (key[j] ^ prefix) < (1u << 21);
+      } else {
+        bin = key[j] & 1023u;
+        counts = (key[j] ^ prefix) < (1u << 10);
+      }
+      atomicAdd(&h[counts ? bin : dummy], 1u);
+      if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();                               // histogram complete
+    // suffix scan from the highest digit down: thread t owns the BPT digits below 2048 - BPT * t
+    uint32_t c[BPT], tot = 0u;
+    {
+      const uint2* hv = reinterpret_cast<const uint2*>(h + NBIN - BPT * (tid + 1));
+#pragma unroll
+      for (int i = 0; i < BPT / 2; ++i) {
+        const uint2 v = hv[BPT / 2 - 1 - i];
+        c[2 * i] = v.y; c[2 * i + 1] = v.x;
+      }
+#pragma unroll
+      for (int b = 0; b < BPT; ++b) tot += c[b];
+    }
+    if (pass == 1) clear(0);                       // for pass 2; its readers have passed a barrier
+    const uint32_t incl = wave_incl_scan(tot, lane);
+    if (lane == 63) sh.wsum[wave] = incl;
+    __syncthreads();
+    uint32_t above = incl - tot;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) above += w < wave ? sh.wsum[w] : 0u;
+    if (above < (uint32_t)need && (uint32_t)need <= above + tot) {   // one thread: its bins hold the k-th best
+#pragma unroll
+      for (int b = 0; b < BPT; ++b) {
+        if (above < (uint32_t)need && (uint32_t)need <= above + c[b]) {
+          sh.pick[0] = (uint32_t)(NBIN - 1 - BPT * tid - b);
+          sh.pick[1] = above;
+          sh.pick[2] = above + c[b] == (uint32_t)need ? 1u : 0u;
+        }
+        above += c[b];
+      }
+    }
+    __syncthreads();
+    prefix |= (uint32_t)__builtin_amdgcn_readfirstlane((int)sh.pick[0]) << shift;
+    need -= __builtin_amdgcn_readfirstlane((int)sh.pick[1]);
+    whole = __builtin_amdgcn_readfirstlane((int)sh.pick[2]) != 0;
+    if (whole) break;                              // uniform; pick is written again only past two barriers
+  }
+
+  // whole: every key >= prefix is taken. Else all three digits are resolved: keys above, and the
+  // first `need` entries of those equal.
+  const uint32_t T = prefix;
+  forget();
+  auto emit = [&](uint64_t m, bool take, uint32_t base, int j) {
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
+    const int p = p0 + 64 * j;
+    if constexpr (LISTS) {
+      if (take) {
+        *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(ckey + list) + (rank << 2)) = key[j];
+        *reinterpret_cast<int32_t*>(reinterpret_cast<char*>(cpos + list) + (rank << 2)) = ch * chunk + p;
+      }
+    } else {
+      if (take) *reinterpret_cast<int32_t*>(o + (rank << 2)) = p < lens ? p + offset : -1;
+    }
+  };
+  auto waves_before = [&](uint32_t mine) {         // the sum of `mine` (per lane) over the waves before this one
+    const uint32_t incl = wave_incl_scan(mine, lane);
+    if (lane == 63) sh.wsum[wave] = incl;          // last read before the final pass barrier
+    __syncthreads();
+    uint32_t before = 0u;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) before += w < wave ? sh.wsum[w] : 0u;
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)before);
+  };
+  if (whole) {
+    uint32_t cnt = 0u;
+#pragma unroll
+    for (int j = 0; j < J; ++j) cnt += key[j] >= T ? 1u : 0u;
+    uint32_t base = waves_before(cnt);
+    uint32_t T2 = T;                               // opaque: the compiler would keep J comparison masks from above
+    asm volatile("" : "+s"(T2));
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const bool take = key[j] >= T2;
+      const uint64_t m = __ballot(take);
+      emit(m, take, base, j);
+      base += (uint32_t)__popcll(m);
+      if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+  } else {
+    uint32_t cnt = 0u;                             // above T << 16 | equal (at most 32,768 of either)
+#pragma unroll
+    for (int j = 0; j < J; ++j) cnt += (key[j] > T ? 0x10000u : 0u) + (key[j] == T ? 1u : 0u);
+    const uint32_t before = waves_before(cnt);
+    uint32_t eq = before & 0xFFFFu, base = (before >> 16) + min(eq, (uint32_t)need);
+    uint32_t T2 = T;                               // opaque, as above
+    asm volatile("" : "+s"(T2));
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const uint64_t e = __ballot(key[j] == T2);
+      const uint32_t er = __builtin_amdgcn_mbcnt_hi((uint32_t)(e >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)e, eq));
+      const bool take = key[j] > T2 || (key[j] == T2 && er < (uint32_t)need);
+      const uint64_t m = __ballot(take);
+      emit(m, take, base, j);
+      base += (uint32_t)__popcll(m);
+      eq += (uint32_t)__popcll(e);
+      if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
 // Rows longer than 32k scores: keys are re-read from memory in every pass.
 __global__ __launch_bounds__(kSelThreads) void topk_kernel(const float* __restrict__ scores, int32_t* __restrict__ out,
                                                            int n, int nb, int k, int start_pos, int ratio,
@@ -346,23 +547,83 @@ int topk_merge_launch(const char* what, const uint32_t* ckey, const int32_t* cpo
 }
 }  // namespace dsv41
 
-// The two-stage form for a row of nb scores: rows longer than one 16-keys-per-thread workgroup
-// holds, k at most half a chunk, and the chunk lists small enough for one register workgroup.
+// How a selection over `rows` rows of nb scores runs.
+struct TopkPlan {
+  bool stripe;         // topk_stripe_kernel (the whole row, or stage 1)
+  int chunks, chunk;   // two stages: per-chunk lists, then a merge (chunks 0: one stage)
+};
+
+constexpr int kStripeMax = 32 * kSelThreads;   // entries of the largest stripe workgroup
+
+// Stripe workgroups win once the chip has rows enough to fill it, and earlier where a row would
+// otherwise go in two stages (single calls, graph-replayed, 1,024-thread register kernel or two
+// stages -> stripe):
+//   4,096 scores, top-512:    256 rows 7.0 -> 7.5 us,   512 rows 9.1 -> 8.3,   8,192 rows 83.1 -> 38.2
+//   10,240 scores, top-2,048: 256 rows 10.4 -> 11.5 us, 512 rows 18.0 -> 13.5, 8,192 rows 238.4 -> 84.5
+//   16,384 scores, top-512:   256 rows 11.1 -> 11.7 us, 512 rows 19.7 -> 15.4, 8,192 rows 271.3 -> 128.5
+//   32,768 scores, top-512:   32 rows 13.9 -> 15.4 us,  64 rows 16.2 -> 15.5,  2,048 rows 194.3 -> 79.9
+// Rows over 32,768 scores go in two stages whose chunks are as few and as even as stripe workgroups
+// can hold (65,536 scores, top-512: 64 rows 20.6 us either way, 128 rows 32.1 -> 21.8 us, 2,048 rows
+// 386 -> 173.5 us).
+//
+// Fewer rows: rows longer than one 16-keys-per-thread workgroup holds go in two stages, with k at
+// most half a chunk and the chunk lists small enough for one register workgroup.
 // For 16 rows of 32,768 scores and k = 1,024 one 32-keys-per-thread workgroup per row is faster
 // on scores already in cache (17.5-19.3 against 19.4-20.2 us), but inside a decode step, reading
 // the scores the scoring kernel has just written, the two stages spread that read over 8
 // workgroups per row and win: the 40-layer fp8 step took 1.163-1.166 ms against 1.190-1.195 ms.
-static bool topk_two_stage(int nb, int k, int* chunks, int* jm, int* chunk) {
-  if (nb <= 16 * kSelThreads || 2 * k > kTopkChunk) return false;
+static TopkPlan topk_plan(int64_t rows, int nb, int k, bool allow_two_stage) {
+  TopkPlan p{false, 0, 0};
+  if (k >= nb) return p;                           // everything is selected
+  if (nb <= kStripeMax) {
+    p.stripe = rows >= 512 || (nb > 16 * kSelThreads && rows >= 64);
+    if (p.stripe) return p;
+  }
+  if (!allow_two_stage || nb <= 16 * kSelThreads) return p;
+  if (nb > kStripeMax && rows >= 128) {
+    const int c = (nb + kStripeMax - 1) / kStripeMax;
+    const int ch = ((nb + c - 1) / c + 63) / 64 * 64;
+    if (k <= ch && (int64_t)c * k <= 32 * kSelThreads && (int64_t)(c - 1) * ch < nb && rows * c < (1ll << 31)) {
+      p.stripe = true;
+      p.chunks = c;
+      p.chunk = ch;
+      return p;
+    }
+  }
+  if (2 * k > kTopkChunk) return p;
   // lists of more than 4,096 entries per row with 4,096-entry chunks: 8,192-entry chunks halve them
   const int ch = (int64_t)((nb + kTopkChunk - 1) / kTopkChunk) * k > 4 * kSelThreads ? 2 * kTopkChunk : kTopkChunk;
   const int c = (nb + ch - 1) / ch;
-  const int64_t m = (int64_t)c * k;
-  if (m > 32 * kSelThreads) return false;
-  *chunks = c;
-  *chunk = ch;
-  *jm = m <= 4 * kSelThreads ? 4 : (m <= 8 * kSelThreads ? 8 : (m <= 16 * kSelThreads ? 16 : 32));
-  return true;
+  if ((int64_t)c * k > 32 * kSelThreads) return p;
+  p.chunks = c;
+  p.chunk = ch;
+  return p;
+}
+
+// Launches topk_stripe_kernel for selections of at most `len` entries on a grid of one workgroup each.
+template <bool LISTS>
+static void launch_stripe(int len, unsigned grid, const float* scores, int32_t* out, int n, int nb, int k,
+                          int start_pos, int ratio, int offset, int chunks, int chunk, uint32_t* ckey, int32_t* cpos,
+                          hipStream_t stream) {
+#define DSV41_STRIPE_CASE(NT_, J_)                                                                                  \
+  if (len <= NT_ * J_) {                                                                                            \
+    hipLaunchKernelGGL((topk_stripe_kernel<NT_, J_, LISTS>), dim3(grid), dim3(NT_), 0, stream, scores, out, n, nb, k, \
+                       start_pos, ratio, offset, chunks, chunk, ckey, cpos);                                        \
+    return;                                                                                                         \
+  }
+  if constexpr (!LISTS) {                          // chunks are longer than half of kStripeMax
+    DSV41_STRIPE_CASE(256, 8)
+    DSV41_STRIPE_CASE(256, 16)
+    DSV41_STRIPE_CASE(256, 24)
+    DSV41_STRIPE_CASE(256, 32)
+    DSV41_STRIPE_CASE(256, 40)
+    DSV41_STRIPE_CASE(512, 24)
+    DSV41_STRIPE_CASE(512, 32)
+  }
+  DSV41_STRIPE_CASE(512, 40)
+  DSV41_STRIPE_CASE(1024, 24)
+  DSV41_STRIPE_CASE(1024, 32)
+#undef DSV41_STRIPE_CASE
 }
 
 static size_t topk_ws_bytes(int64_t rows, int chunks, int k) {
@@ -382,8 +643,9 @@ static int topk_launch(const char* what, const float* scores, int32_t* out, int6
   if (rows == 0 || k == 0) return 0;
   const dim3 grid((unsigned)rows), block(kSelThreads);
   const int vec = (nb % 4 == 0 && aligned16(scores)) ? 1 : 0;
-  int chunks = 0, jm = 0, chunk = 0;
-  if (allow_two_stage && topk_two_stage(nb, k, &chunks, &jm, &chunk)) {
+  const TopkPlan plan = topk_plan(rows, nb, k, allow_two_stage);
+  if (plan.chunks) {
+    const int chunks = plan.chunks, chunk = plan.chunk;
     const size_t need = topk_ws_bytes(rows, chunks, k);
     DSV41_REQUIRE(workspace && workspace_bytes >= need, DSV41_E_WORKSPACE, "%s: workspace of %zu bytes needed", what,
                   need);
@@ -391,15 +653,23 @@ static int topk_launch(const char* what, const float* scores, int32_t* out, int6
     DSV41_REQUIRE(rows * chunks < (1ll << 31), DSV41_E_ARG, "%s: too many row chunks", what);
     uint32_t* ckey = reinterpret_cast<uint32_t*>(workspace);
     int32_t* cpos = reinterpret_cast<int32_t*>(reinterpret_cast<uint8_t*>(workspace) + need / 2);
-    if (chunk == kTopkChunk)
-      hipLaunchKernelGGL(topk_chunk_kernel<kTopkChunk / kSelThreads>, dim3((unsigned)(rows * chunks)), block, 0, stream,
-                         scores, ckey, cpos, nb, k, chunks, vec);
+    const dim3 cgrid((unsigned)(rows * chunks));
+    if (plan.stripe)
+      launch_stripe<true>(chunk, cgrid.x, scores, out, n, nb, k, start_pos, ratio, offset, chunks, chunk, ckey, cpos,
+                          stream);
+    else if (chunk == kTopkChunk)
+      hipLaunchKernelGGL(topk_chunk_kernel<kTopkChunk / kSelThreads>, cgrid, block, 0, stream, scores, ckey, cpos, nb, k,
+                         chunks, vec);
     else
-      hipLaunchKernelGGL(topk_chunk_kernel<2 * kTopkChunk / kSelThreads>, dim3((unsigned)(rows * chunks)), block, 0,
-                         stream, scores, ckey, cpos, nb, k, chunks, vec);
+      hipLaunchKernelGGL(topk_chunk_kernel<2 * kTopkChunk / kSelThreads>, cgrid, block, 0, stream, scores, ckey, cpos,
+                         nb, k, chunks, vec);
     int rc = check_launch(what);
     if (rc) return rc;
     return topk_merge_launch(what, ckey, cpos, out, rows, n, nb, k, chunks, chunk, start_pos, ratio, offset, stream);
+  }
+  if (plan.stripe) {
+    launch_stripe<false>(nb, grid.x, scores, out, n, nb, k, start_pos, ratio, offset, 1, nb, nullptr, nullptr, stream);
+    return check_launch(what);
   }
   if (nb <= 4 * kSelThreads)
     hipLaunchKernelGGL(topk_reg_kernel<4>, grid, block, 0, stream, scores, out, n, nb, k, start_pos, ratio, offset, vec);
@@ -425,8 +695,8 @@ extern "C" int dsv41_topk_select(const float* scores, int32_t* out, int64_t rows
 extern "C" size_t dsv41_topk_workspace_bytes(int64_t rows, int32_t nb, int32_t topk) {
   if (rows <= 0 || nb <= 0 || topk <= 0) return 0;
   const int k = topk < nb ? topk : nb;
-  int chunks = 0, jm = 0, chunk = 0;
-  return topk_two_stage(nb, k, &chunks, &jm, &chunk) ? topk_ws_bytes(rows, chunks, k) : 0;
+  const TopkPlan p = topk_plan(rows, nb, k, true);
+  return p.chunks ? topk_ws_bytes(rows, p.chunks, k) : 0;
 }
 
 extern "C" int dsv41_topk_select_ws(const float* scores, int32_t* out, int64_t rows, int32_t n, int32_t nb,

@@ -939,9 +939,9 @@ def topk_workspace_bytes(rows, nb, topk) -> int:
 
 
 def topk_select(scores, topk, start_pos, ratio, offset, workspace=None, out=None):
-    """scores [b, n, nb] fp32 -> int32 [b, n, min(topk, nb)] (into `out` when given). Rows longer
-    than 16384 scores (k <= 2048) are selected in two stages through a uint8 workspace of
-    topk_workspace_bytes(...) bytes, allocated when it is omitted or too small."""
+    """scores [b, n, nb] fp32 -> int32 [b, n, min(topk, nb)] (into `out` when given). Long rows are
+    selected in two stages through a uint8 workspace of topk_workspace_bytes(...) bytes, allocated
+    when it is omitted or too small."""
     name = "dsv41_topk_select_ws"
     _gpu(name, scores, workspace, out)
     _contig(name, scores)

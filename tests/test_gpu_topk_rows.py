@@ -1,0 +1,68 @@
+"""Selection over many rows (a chunk's queries) against the same rows selected a few at a time, which take other kernels."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _scores(rows, nb, kind):
+    g = torch.Generator(device="cuda").manual_seed(rows + nb)
+    x = torch.randn(rows, 1, nb, generator=g, device="cuda")
+    if kind == "ties":                   # five values, both zeros among them
+        x = (x * 1.2).round().clamp(-2, 2)
+        x = torch.where(x == 0, torch.where(torch.rand(x.shape, generator=g, device="cuda") < 0.5, -0.0, 0.0), x)
+    elif kind == "masked":               # most entries -inf, some rows with fewer finite ones than k
+        x.masked_fill_(torch.rand(x.shape, generator=g, device="cuda") < 0.97, -float("inf"))
+        x[:3] = -float("inf")
+    elif kind == "odd":                  # infinities and NaNs of both signs, the all-ones one included
+        bits = x.view(torch.int32)
+        pick = torch.randint(0, 12, x.shape, generator=g, device="cuda")
+        for i, v in enumerate((0x7F800000, -0x800000, 0x7FC00000, -0x400000, -1)):
+            bits.masked_fill_(pick == i, v)
+    return x.contiguous()
+
+
+@pytest.mark.parametrize("rows,nb,k", [
+    (512, 2, 1), (513, 65, 64), (512, 2048, 512), (600, 2049, 2048), (512, 4096, 1), (512, 4097, 512),
+    (512, 6145, 6144), (512, 8193, 777), (530, 10240, 2048), (512, 10241, 512), (512, 12289, 512), (512, 16384, 1024),
+    (64, 16385, 512), (70, 20481, 2048), (64, 24577, 512), (64, 32768, 4096),
+    (128, 32769, 512),                   # two chunks, the second a little shorter
+    (130, 65536, 2048), (128, 65600, 512),
+    (128, 98305, 4096),                  # four chunks
+])
+@pytest.mark.parametrize("kind", ["normal", "ties", "masked", "odd"])
+def test_rows_equal_few_rows(gpu, rows, nb, k, kind):
+    from dsv41 import _abi
+    x = _scores(rows, nb, kind)
+    start = nb - nb // 7                 # the last positions are past the queries' visibility
+    got = _abi.topk_select(x, k, start, 1, 5)
+    few = torch.cat([_abi.topk_select(x[i:i + 31].contiguous(), k, start, 1, 5) for i in range(0, rows, 31)])
+    assert torch.equal(got, few)
+
+
+def test_rows_of_several_queries(gpu):
+    """Visibility follows the query, row % n, also with rows of several sequences and k >= nb."""
+    from dsv41 import _abi
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(3, 211, 900, generator=g, device="cuda")
+    for k in (100, 900, 2000):
+        got = _abi.topk_select(x, k, 700, 2, 9)
+        few = torch.cat([_abi.topk_select(x[:, i:i + 1].contiguous(), k, 700 + i, 2, 9) for i in range(211)], 1)
+        assert torch.equal(got, few)
+
+
+def test_workspace_matches_the_route(gpu):
+    """Rows that one workgroup selects need no workspace; longer ones state theirs and refuse less."""
+    from dsv41 import _abi
+    assert _abi.topk_workspace_bytes(2048, 32768, 512) == 0
+    need = _abi.topk_workspace_bytes(128, 65536, 512)
+    assert need == 2 * 128 * 2 * 512 * 4
+    x = torch.randn(128, 1, 65536, device="cuda")
+    out = torch.empty(128, 1, 512, dtype=torch.int32, device="cuda")
+    small = torch.empty(need - 256, dtype=torch.uint8, device="cuda")
+    with pytest.raises(ValueError):
+        _abi._call("dsv41_topk_select_ws", _abi._ptr(x), _abi._ptr(out), 128, 1, 65536, 512, 70000, 1, 0,
+                   _abi._ptr(small), small.numel(), _abi._stream(x))
