@@ -1,0 +1,288 @@
+// The compressor's two projections, deepseek_v41_mlx/compressor.py:59-61: kv = x wkv^T and
+// score = x wgate^T with float32 weights, in float32, for bf16 activations x.
+//
+//   y0[m, j] = sum_k x[m, k] * w0[j, k],  y1[m, j] = sum_k x[m, k] * w1[j, k]
+//
+// On the bf16 matrix cores without giving up any of the 24 bits of a weight: a float32 w is cut, by
+// truncation, into three bf16 numbers of 8 significand bits each, w = h + m + l exactly, and the
+// three products with the (already bf16) activation are exact in the MFMA, which adds them up in
+// float32. Relative error (2-norm) against the float64 result, k = 5120, library float32 GEMM and this
+// one: 64 rows 6.4e-7 and 2.0e-7, 1,024 rows 1.28e-6 and 5.5e-7, 8,192 rows 1.28e-6 and 7.9e-7.
+//
+// Bound by the matrix cores at chunk row counts (3 x 2 rows k n multiply-adds on the bf16 rate, a
+// sixteenth of which is what float32 MFMAs reach) and by the weight stream (4 bytes each) at decode
+// row counts. Both projections, k = 5120, n = 512 + 512, against the library (x widened to float32,
+// then two float32 GEMMs): 8,191 rows 616 -> 236 us (1,090 TFLOP/s of bf16 products), 2,048 rows 173 ->
+// 81 us, 64 rows 28.6 -> 15.5 us, 1 row 26.5 -> 13.6 us.
+//
+// A workgroup owns TR weight rows (of the two weights stacked) x TM activation rows and walks 64
+// channels per step, double-buffered. The activations arrive by LDS copies; the weights pass through
+// registers, where each is cut once per workgroup, and lie in LDS as three bf16 planes, all in the
+// XOR-swizzled rows that the fragment reads take without bank conflicts. The contraction is cut into
+// `splits` ranges where the tiles alone would not fill the chip; then each range's float32 partial
+// goes to the workspace and a second kernel adds them in range order.
+#include "mfma.h"
+
+namespace dsv41 {
+
+struct ProjArgs {
+  const bf16_t* x;                       // [rows, k]
+  const float *w0, *w1;                  // [n0, k], [n - n0, k]
+  float *y0, *y1;                        // [rows, n0], [rows, n - n0]
+  float* part;                           // [splits, rows, n] partial sums (splits > 1)
+  int rows, k, n, n0, splits;
+};
+
+// 16-byte chunk c of a 128-byte tile row (64 bf16) sits at slot c ^ proj_swz(row): a fragment read
+// takes one chunk of 16 consecutive rows and no two of its lanes share a bank.
+__device__ __forceinline__ int proj_swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+
+// The three bf16 planes of four weights, as packed pairs (even channel low): the upper 16 bits of
+// what is left after each plane. Every difference is exact (at most 16, then 8 bits remain).
+struct Planes {
+  uint2 p[3];
+};
+__device__ __forceinline__ Planes cut_weights(const float4 w) {
+  float r[4] = {w.x, w.y, w.z, w.w};
+  Planes o;
+#pragma unroll
+  for (int s = 0; s < 3; ++s) {
+    uint32_t u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      u[i] = __float_as_uint(r[i]);
+      r[i] = r[i] - __uint_as_float(u[i] & 0xFFFF0000u);
+    }
+    o.p[s] = make_uint2(__builtin_amdgcn_perm(u[1], u[0], 0x07060302u), __builtin_amdgcn_perm(u[3], u[2], 0x07060302u));
+  }
+  return o;
+}
+
+// Infinities: an infinite weight leaves NaN behind its first plane, and an infinite activation
+// meets planes that are 0, so a result that should be infinite comes out NaN. A NaN result is
+// therefore formed again in plain float32 (never taken with finite inputs).
+__device__ __noinline__ float plain_dot(const bf16_t* x, const float* w, int k) {
+  float s = 0.0f;
+  for (int i = 0; i < k; ++i) s += bf2f(x[i]) * w[i];
+  return s;
+}
+__device__ __forceinline__ void store_proj(const ProjArgs& a, int m, int j, f32x4 v) {   // columns j .. j + 3 of row m
+  const bool second = j >= a.n0;
+  const int jj = second ? j - a.n0 : j;
+  if (__any(v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3])) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (v[i] != v[i])
+        v[i] = plain_dot(a.x + (int64_t)m * a.k, (second ? a.w1 : a.w0) + (int64_t)(jj + i) * a.k, a.k);
+  }
+  float* y = second ? a.y1 + (int64_t)m * (a.n - a.n0) : a.y0 + (int64_t)m * a.n0;
+  *reinterpret_cast<f32x4*>(y + jj) = v;
+}
+
+// A GR x GM grid of waves, each 16 WR weight rows x 16 WM activation rows.
+template <int WR, int WM, int GR, int GM>
+struct ProjCfg {
+  static constexpr int NWV = GR * GM, NT = 64 * NWV;
+  static constexpr int TR = 16 * WR * GR, TM = 16 * WM * GM;
+  static constexpr int BK = 64, RB = BK * 2;
+  static constexpr int PLANE = TR * RB, STAGE = 3 * PLANE + TM * RB, LDS = 2 * STAGE;
+  static constexpr int WL = TR / (4 * NWV);           // 1 KB weight loads per wave and step (4 rows of 256 bytes)
+  static constexpr int XL = TM / (8 * NWV);           // 1 KB activation copies per wave and step (8 rows of 128 bytes)
+  static_assert(WL * 4 * NWV == TR && XL * 8 * NWV == TM, "whole load instructions per wave");
+  static_assert(LDS <= 160 * 1024, "LDS budget");
+};
+
+template <int WR, int WM, int GR, int GM>
+__global__ __launch_bounds__(64 * GR * GM, (ProjCfg<WR, WM, GR, GM>::LDS <= 80 * 1024) ? 4 : 2) void proj_f32_kernel(
+    ProjArgs a) {
+  using C = ProjCfg<WR, WM, GR, GM>;
+  __shared__ __align__(16) uint8_t lds[C::LDS];       // 2 x [h plane][m plane][l plane][activations]
+  const int rtiles = a.n / C::TR;
+  // consecutive tiles on one XCD, the weight tile fastest: the workgroups that read one activation
+  // tile share that XCD's L2
+  const int total = (int)gridDim.x;
+  const int tile = total % 8 ? (int)blockIdx.x : ((int)blockIdx.x % 8) * (total / 8) + (int)blockIdx.x / 8;
+  const int rt = tile % rtiles, sp = (tile / rtiles) % a.splits, mt = tile / (rtiles * a.splits);
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wr = (wave % GR) * 16 * WR, wm = (wave / GR) * 16 * WM;   // this wave's block
+  const int kr = a.k / a.splits;                      // channels of this range
+  // weights: wave w loads tile rows w TR/NWV + 4 j + g, lane l16 the channels 4 l16 .. + 3 of a step
+  const float* wsrc[C::WL];
+  int wdst[C::WL];
+#pragma unroll
+  for (int j = 0; j < C::WL; ++j) {
+    const int row = wave * (C::TR / C::NWV) + 4 * j + g;
+    const int all = rt * C::TR + row;
+    const float* base = all < a.n0 ? a.w0 + (int64_t)all * a.k : a.w1 + (int64_t)(all - a.n0) * a.k;
+    wsrc[j] = base + (int64_t)sp * kr + 4 * l16;
+    wdst[j] = row * C::RB + (((l16 >> 1) ^ proj_swz(row)) << 4) + 8 * (l16 & 1);
+  }
+  uint64_t xsrc[C::XL];
+#pragma unroll
+  for (int j = 0; j < C::XL; ++j) {
+    const int row = wave * (C::TM / C::NWV) + 8 * j + (lane >> 3);
+    const int64_t m = min(mt * C::TM + row, a.rows - 1);              // rows past the end: not stored
+    xsrc[j] = reinterpret_cast<uint64_t>(a.x + m * a.k + (int64_t)sp * kr + 8 * ((lane & 7) ^ proj_swz(row)));
+  }
+  const uint32_t lds0 = lds_offset(lds);
+  auto issue_x = [&](int buf, int kt) {
+    const uint32_t dst = (uint32_t)__builtin_amdgcn_readfirstlane(
+        (int)(lds0 + (uint32_t)(buf * C::STAGE + 3 * C::PLANE) + (uint32_t)(wave * (C::TM / C::NWV) * C::RB)));
+#pragma unroll
+    for (int j = 0; j < C::XL; ++j) dma16_vaddr(xsrc[j] + (uint64_t)kt * C::RB, dst + j * 1024);
+  };
+  float4 wreg[C::WL];
+  auto load_w = [&](int kt) {
+#pragma unroll
+    for (int j = 0; j < C::WL; ++j) wreg[j] = *reinterpret_cast<const float4*>(wsrc[j] + kt * C::BK);
+  };
+  auto store_w = [&](int buf) {
+#pragma unroll
+    for (int j = 0; j < C::WL; ++j) {
+      const Planes p = cut_weights(wreg[j]);
+#pragma unroll
+      for (int s = 0; s < 3; ++s) *reinterpret_cast<uint2*>(lds + buf * C::STAGE + s * C::PLANE + wdst[j]) = p.p[s];
+    }
+  };
+  auto frag = [&](const uint8_t* t, int row, int chunk) {
+    return ld_bf16x8(t + row * C::RB + ((chunk ^ proj_swz(row)) << 4));
+  };
+
+  f32x4 acc[WR][WM];
+#pragma unroll
+  for (int i = 0; i < WR; ++i)
+#pragma unroll
+    for (int j = 0; j < WM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int nk = kr / C::BK;
+  issue_x(0, 0);
+  load_w(0);
+  store_w(0);
+  for (int kt = 0; kt < nk; ++kt) {
+    const int buf = kt & 1;
+    wait_vmcnt<0>();                                  // this wave's activation copies of step kt
+    __syncthreads();                                  // step kt is in LDS; step kt - 1's buffer is free
+    const bool more = kt + 1 < nk;
+    if (more) {
+      issue_x(buf ^ 1, kt + 1);                       // copies first: the wait for the weights covers them
+      load_w(kt + 1);
+    }
+    const uint8_t* wt = lds + buf * C::STAGE;
+    const uint8_t* xt = wt + 3 * C::PLANE;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      bf16x8 bx[WM];
+#pragma unroll
+      for (int j = 0; j < WM; ++j) bx[j] = frag(xt, wm + 16 * j + l16, 4 * ks + g);
+#pragma unroll
+      for (int s = 2; s >= 0; --s) {                  // the smallest plane first
+        bf16x8 af[WR];
+#pragma unroll
+        for (int i = 0; i < WR; ++i) af[i] = frag(wt + s * C::PLANE, wr + 16 * i + l16, 4 * ks + g);
+#pragma unroll
+        for (int i = 0; i < WR; ++i)
+#pragma unroll
+          for (int j = 0; j < WM; ++j) acc[i][j] = mfma16x16x32(af[i], bx[j], acc[i][j]);
+      }
+    }
+    if (more) store_w(buf ^ 1);                       // the next step's weights, cut, while the MFMAs drain
+  }
+
+#pragma unroll
+  for (int j = 0; j < WM; ++j) {
+    const int m = mt * C::TM + wm + 16 * j + l16;
+    if (m >= a.rows) continue;
+#pragma unroll
+    for (int i = 0; i < WR; ++i) {
+      const int col = rt * C::TR + wr + 16 * i + 4 * g;
+      if (a.splits > 1) *reinterpret_cast<f32x4*>(a.part + ((int64_t)sp * a.rows + m) * a.n + col) = acc[i][j];
+      else store_proj(a, m, col, acc[i][j]);
+    }
+  }
+}
+
+// y[m, j] = sum over the ranges, in order, of part[s][m][j]; four outputs per thread.
+__global__ __launch_bounds__(256) void proj_reduce_kernel(ProjArgs a) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const int64_t total = (int64_t)a.rows * a.n;
+  if (i >= total) return;
+  f32x4 acc = *reinterpret_cast<const f32x4*>(a.part + i);
+  for (int s = 1; s < a.splits; ++s) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(a.part + s * total + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] += v[e];
+  }
+  const int m = (int)(i / a.n);
+  store_proj(a, m, (int)(i - (int64_t)m * a.n), acc);
+}
+
+template <int WR, int WM, int GR, int GM>
+static void launch_proj(const ProjArgs& a, hipStream_t stream) {
+  using C = ProjCfg<WR, WM, GR, GM>;
+  const int64_t tiles = (int64_t)(a.n / C::TR) * a.splits * ((a.rows + C::TM - 1) / C::TM);
+  hipLaunchKernelGGL((proj_f32_kernel<WR, WM, GR, GM>), dim3((unsigned)tiles), dim3(C::NT), 0, stream, a);
+}
+
+struct ProjPlan {
+  int tr, tm, splits;
+};
+
+// Tiles as large as still give the chip a workgroup per CU (8 weight tiles at n = 1024), then as many
+// contraction ranges as fit one round of 256 workgroups: large tiles cut and read a weight for more
+// rows, short ranges fill the chip when rows are few.
+static ProjPlan proj_plan(int rows, int k, int n) {
+  ProjPlan p{128, 256, 1};
+  if (rows <= 32) { p.tr = 32; p.tm = 32; }
+  else if (rows <= 128) { p.tr = 64; p.tm = 64; }
+  else if (rows <= 1024) p.tm = 64;
+  else if (rows <= 4096) p.tm = 128;
+  const int64_t tiles = (int64_t)(n / p.tr) * ((rows + p.tm - 1) / p.tm);
+  for (int s = 2; s <= 40; ++s)                        // ranges of whole 64-channel steps, one wave of the chip
+    if (k % (64 * s) == 0 && tiles * s <= 256) p.splits = s;
+  return p;
+}
+
+}  // namespace dsv41
+
+using namespace dsv41;
+
+extern "C" size_t dsv41_linear_f32_pair_workspace_bytes(int32_t rows, int32_t k, int32_t n0, int32_t n1) {
+  if (rows <= 0 || k <= 0 || n0 <= 0 || n1 < 0) return 0;
+  const int n = n0 + n1;
+  if (k % 64 || n0 % 128 || n1 % 128) return 0;
+  const ProjPlan p = proj_plan(rows, k, n);
+  return p.splits > 1 ? (size_t)p.splits * (size_t)rows * (size_t)n * sizeof(float) : 0;
+}
+
+extern "C" int dsv41_linear_f32_pair(const void* x, const float* w0, const float* w1, float* y0, float* y1,
+                                     void* workspace, size_t workspace_bytes, int32_t rows, int32_t k, int32_t n0,
+                                     int32_t n1, int32_t dtype, hipStream_t stream) {
+  const char* what = "dsv41_linear_f32_pair";
+  DSV41_REQUIRE(x && w0 && w1 && y0 && y1, DSV41_E_ARG, "%s: null tensor", what);
+  DSV41_REQUIRE(dtype == DSV41_BF16, DSV41_E_DTYPE, "%s: bf16 activations only (dtype %d)", what, dtype);
+  DSV41_REQUIRE(rows >= 0 && k > 0 && n0 > 0 && n1 > 0 && (int64_t)n0 + n1 < (1 << 24), DSV41_E_ARG, "%s: bad sizes", what);
+  DSV41_REQUIRE(k % 64 == 0 && n0 % 128 == 0 && n1 % 128 == 0, DSV41_E_SHAPE,
+                "%s: k = %d must be a multiple of 64, n0 = %d and n1 = %d of 128", what, k, n0, n1);
+  DSV41_REQUIRE(aligned16(x) && aligned16(w0) && aligned16(w1) && aligned16(y0) && aligned16(y1), DSV41_E_ARG,
+                "%s: tensors must be 16-byte aligned", what);
+  if (rows == 0) return 0;
+  const ProjPlan p = proj_plan(rows, k, n0 + n1);
+  DSV41_REQUIRE((int64_t)((n0 + n1) / p.tr) * p.splits * (((int64_t)rows + p.tm - 1) / p.tm) < (1ll << 31), DSV41_E_ARG,
+                "%s: too many tiles", what);
+  const size_t need = dsv41_linear_f32_pair_workspace_bytes(rows, k, n0, n1);
+  DSV41_REQUIRE(workspace_bytes >= need && (need == 0 || (workspace && aligned16(workspace))), DSV41_E_WORKSPACE,
+                "%s: workspace of %zu bytes needed, %zu given", what, need, workspace_bytes);
+  ProjArgs a{static_cast<const bf16_t*>(x), w0, w1, y0, y1, static_cast<float*>(workspace), rows, k, n0 + n1, n0,
+             p.splits};
+  if (p.tr == 32) launch_proj<1, 1, 2, 2>(a, stream);
+  else if (p.tr == 64) launch_proj<1, 2, 4, 2>(a, stream);
+  else if (p.tm == 64) launch_proj<2, 2, 4, 2>(a, stream);
+  else if (p.tm == 128) launch_proj<2, 4, 4, 2>(a, stream);
+  else launch_proj<4, 4, 2, 4>(a, stream);
+  int rc = check_launch(what);
+  if (rc || p.splits <= 1) return rc;
+  const int64_t quads = (int64_t)rows * a.n / 4;
+  hipLaunchKernelGGL(proj_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, a);
+  return check_launch(what);
+}

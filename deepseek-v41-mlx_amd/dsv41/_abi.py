@@ -98,6 +98,8 @@ _SIGNATURES = {
     "dsv41_linear_rows_workspace_bytes": [_i32, _i32, _i32],
     "dsv41_linear_rows": [_c_p, _c_p, _c_p, _c_p, _sz, _i32, _i32, _i32, _i32, _i32, _c_p],
     "dsv41_linear_rows_pair": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _sz, _i32, _i32, _i32, _i32, _i32, _i32, _c_p],
+    "dsv41_linear_f32_pair_workspace_bytes": [_i32, _i32, _i32, _i32],
+    "dsv41_linear_f32_pair": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _sz, _i32, _i32, _i32, _i32, _i32, _c_p],
     "dsv41_comp_write_fp8": [_c_p, _c_p, _i64, _c_p, _i64, _i32, _c_p, _c_p, _i32, _i32, _i32, _i32, _i32, _i32,
                              _i32, _c_p],
     "dsv41_index_key_publish_fp8": [_c_p, _c_p, _i64, _c_p, _i64, _i32, _c_p, _c_p, _c_p, _i32, _i32, _i32, _i32,
@@ -112,6 +114,7 @@ _SIGNATURES = {
 _RESTYPES = {
     "dsv41_sparse_mla_workspace_bytes": _sz,
     "dsv41_linear_rows_workspace_bytes": _sz,
+    "dsv41_linear_f32_pair_workspace_bytes": _sz,
     "dsv41_topk_workspace_bytes": _sz,
     "dsv41_indexer_topk_workspace_bytes": _sz,
     "dsv41_version": ctypes.c_char_p,
@@ -385,6 +388,27 @@ def window_idx(wp, n, window, device):
 
 
 # ---------------------------------------------------------------------------- compressor
+
+
+def linear_f32_pair(x, w0, w1, workspace=None):
+    """(x @ w0^T, x @ w1^T) in float32 for bf16 x [..., k] and float32 weights [n, k]: the compressor's
+    two projections (compressor.py:59-61), the weights' 24 bits kept (dsv41_linear_f32_pair)."""
+    name = "dsv41_linear_f32_pair"
+    _gpu(name, x, w0, w1)
+    _contig(name, x, w0, w1)
+    if x.dtype != torch.bfloat16 or w0.dtype != torch.float32 or w1.dtype != torch.float32:
+        raise ValueError(f"{name}: x must be bfloat16, the weights float32")
+    if w0.dim() != 2 or w1.dim() != 2 or not w0.shape[1] == w1.shape[1] == x.shape[-1]:
+        raise ValueError(f"{name}: x {tuple(x.shape)}, w0 {tuple(w0.shape)} and w1 {tuple(w1.shape)} do not contract")
+    k, n0, n1 = w0.shape[1], w0.shape[0], w1.shape[0]
+    rows = x.numel() // k
+    y0 = torch.empty(*x.shape[:-1], n0, dtype=torch.float32, device=x.device)
+    y1 = torch.empty(*x.shape[:-1], n1, dtype=torch.float32, device=x.device)
+    need = lib().dsv41_linear_f32_pair_workspace_bytes(rows, k, n0, n1)
+    ws = _ws(name, workspace, need, x.device)
+    _call(name, _ptr(x), _ptr(w0), _ptr(w1), _ptr(y0), _ptr(y1), _ptr(ws), need, rows, k, n0, n1,
+          dtype_code(x, name), _stream(x))
+    return y0, y1
 
 
 def compress_pool(kv, score, kv_state, score_state, norm_w, ratio, start_pos, eps, dtype):

@@ -1,7 +1,7 @@
 """Learned KV compression (deepseek_v41_mlx/compressor.py:36-88) on the GPU.
 
-* ratio > 1 (owner layers): ``kv = x @ wkv^T`` and ``score = x @ wgate^T`` in fp32 (the two
-  projections are torch GEMMs), then one HIP kernel prepends the carried partial group,
+* ratio > 1 (owner layers): ``kv = x @ wkv^T`` and ``score = x @ wgate^T`` in fp32 (bf16 activations:
+  one kernel for both, dsv41_linear_f32_pair; others: torch GEMMs), then one HIP kernel prepends the carried partial group,
   pools every completed group with a per-channel softmax over the ratio axis, RMSNorms the
   pooled vector and stores the new remainder back into ``CompressorState``;
 * ratio == 1: a plain projection followed by the norm.
@@ -18,6 +18,14 @@ import torch.nn.functional as F
 from . import _abi
 from .config import ModelArgs
 from .layers import RMSNorm
+
+
+def _exact_weights_ok(x: torch.Tensor, w0: torch.Tensor, w1: torch.Tensor) -> bool:
+    """The shapes and dtypes dsv41_linear_f32_pair takes: bf16 activations and float32 weights in whole
+    tiles (64 channels, 128 weight rows)."""
+    return (x.dtype == torch.bfloat16 and x.is_cuda and w0.dtype == w1.dtype == torch.float32 and x.shape[-1] % 64 == 0
+            and w0.shape[0] % 128 == 0 and w1.shape[0] % 128 == 0 and w0.is_contiguous() and w1.is_contiguous()
+            and w0.data_ptr() % 16 == 0 and w1.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
 
 
 class Compressor(torch.nn.Module):
@@ -37,9 +45,13 @@ class Compressor(torch.nn.Module):
     def forward(self, x: torch.Tensor, start_pos: int, comp_state) -> torch.Tensor | None:
         if self.ratio == 1:
             return self.norm(self.wkv(x))
-        xf = x.float()
-        kv = F.linear(xf, self.wkv.weight)
-        score = F.linear(xf, self.wgate.weight)
+        w0, w1 = self.wkv.weight, self.wgate.weight
+        if _exact_weights_ok(x, w0, w1):
+            kv, score = _abi.linear_f32_pair(x.contiguous(), w0, w1)
+        else:
+            xf = x.float()
+            kv = F.linear(xf, w0)
+            score = F.linear(xf, w1)
         return _abi.compress_pool(kv, score, comp_state.kv_state, comp_state.score_state,
                                   self.norm.weight, self.ratio, start_pos, self.norm.eps, x.dtype)
 

@@ -144,6 +144,17 @@ int dsv41_compress_pool(const float* kv, const float* score, float* kv_state, fl
                         int32_t ratio, int32_t start_pos, float eps, int32_t dtype,
                         hipStream_t stream);
 
+/* The compressor's two float32 projections, deepseek_v41_mlx/compressor.py:59-61 (ratio > 1):
+ * y0 = x w0^T [rows, n0] and y1 = x w1^T [rows, n1] in float32, for bf16 x [rows, k] and float32
+ * weights w0 [n0, k], w1 [n1, k]. Each weight enters the bf16 matrix cores as three bf16 numbers whose
+ * sum it is exactly, so products are exact and sums float32. k a multiple of 64, n0 and n1 of 128;
+ * dtype (of x) is BF16. The workspace is dsv41_linear_f32_pair_workspace_bytes(...) bytes, 16-byte
+ * aligned (0: none). */
+size_t dsv41_linear_f32_pair_workspace_bytes(int32_t rows, int32_t k, int32_t n0, int32_t n1);
+int dsv41_linear_f32_pair(const void* x, const float* w0, const float* w1, float* y0, float* y1,
+                          void* workspace, size_t workspace_bytes, int32_t rows, int32_t k, int32_t n0,
+                          int32_t n1, int32_t dtype, hipStream_t stream);
+
 /* The compressed-cache write of Attention.__call__, deepseek_v41_mlx/attention.py:157-163:
  * comp_kv[b, g0 + j] <- fake_quant_fp4_e4m3(rope_tail(latents[b, j], position (g0+j)*ratio), 16)
  * for latents [bsz, g, dim]; comp_kv has `cache_bstride` elements per batch row. */
