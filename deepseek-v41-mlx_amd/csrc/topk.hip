@@ -244,12 +244,19 @@ __global__ __launch_bounds__(kSelThreads) void topk_merge_kernel(const uint32_t*
 //
 // Entries past the row's end have key 0, below every real key but the all-ones NaN's, whose
 // entries all precede them: they are never taken (k < nb: there are enough real entries).
+//
+// The first histogram leaves -inf out. Masked and not yet visible entries are most of many rows, and
+// their additions to one bin went one lane at a time; where the k-th best is itself -inf (a query that
+// sees fewer than k entries) the row is done after that histogram. 2,048 masked rows x 32,768, half of
+// each -inf: 172 -> 86 us; a causal 8,192 x 10,240 chunk's top-2,048 104.5 -> 88 us.
 template <int NT>
 struct StripeShared {
   uint32_t hist[2][2048 + 64];   // the last 64 words: what a pass does not count
   uint32_t wsum[NT / 64];
   uint32_t pick[3];
 };
+
+constexpr uint32_t kNegInfKey = 0x007FFFFFu;     // order_key(-INFINITY)
 
 // LISTS: stage 1 of the two-stage selection (below) over `chunks` chunks of `chunk` entries per row:
 // workgroup (row, chunk) writes its chunk's best min(k, count) as (order key, position).
@@ -307,19 +314,44 @@ __global__ __launch_bounds__(NT, 8) void topk_stripe_kernel(
   uint32_t prefix = 0u;                            // resolved top bits of the k-th best key, in place
   int need = k;                                    // entries still to take from the prefix's bin
   bool whole = false;                              // the bin holds exactly `need` entries
+  const uint32_t dummy = NBIN + lane;
+  uint32_t c[BPT], tot, incl;
+  // suffix scan from the highest digit down: thread t owns the BPT digits below 2048 - BPT * t
+  auto scan = [&](const uint32_t* h) {
+    const uint2* hv = reinterpret_cast<const uint2*>(h + NBIN - BPT * (tid + 1));
+#pragma unroll
+    for (int i = 0; i < BPT / 2; ++i) {
+      const uint2 v = hv[BPT / 2 - 1 - i];
+      c[2 * i] = v.y; c[2 * i + 1] = v.x;
+    }
+    tot = 0u;
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) tot += c[b];
+    incl = wave_incl_scan(tot, lane);
+    if (lane == 63) sh.wsum[wave] = incl;
+    __syncthreads();
+  };
+  auto wave_total = [&]() {
+    uint32_t t = 0u;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) t += sh.wsum[w];
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)t);
+  };
 #pragma unroll
   for (int pass = 0; pass < 3; ++pass) {
     const int shift = pass == 0 ? 21 : (pass == 1 ? 10 : 0);
     uint32_t* h = sh.hist[pass & 1];
-    const uint32_t dummy = NBIN + lane;
     forget();
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       uint32_t bin;
       bool counts;
       if (pass == 0) {
+        // -inf (masked or not yet visible entries, often most of a row) stays out: one bin would
+        // take its additions one lane at a time. So do the keys below it (NaNs with the sign set)
+        // and the entries past the end, key 0.
         bin = key[j] >> 21;
-        counts = p0 + 64 * j < nb;
+        counts = key[j] > kNegInfKey;
       } else if (pass == 1) {
         bin = (key[j] >> 10) & 2047u;
         counts = (key[j] ^ prefix) < (1u << 21);
@@ -331,22 +363,40 @@ __global__ __launch_bounds__(NT, 8) void topk_stripe_kernel(
       if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();                               // histogram complete
-    // suffix scan from the highest digit down: thread t owns the BPT digits below 2048 - BPT * t
-    uint32_t c[BPT], tot = 0u;
-    {
-      const uint2* hv = reinterpret_cast<const uint2*>(h + NBIN - BPT * (tid + 1));
-#pragma unroll
-      for (int i = 0; i < BPT / 2; ++i) {
-        const uint2 v = hv[BPT / 2 - 1 - i];
-        c[2 * i] = v.y; c[2 * i + 1] = v.x;
-      }
-#pragma unroll
-      for (int b = 0; b < BPT; ++b) tot += c[b];
-    }
     if (pass == 1) clear(0);                       // for pass 2; its readers have passed a barrier
-    const uint32_t incl = wave_incl_scan(tot, lane);
-    if (lane == 63) sh.wsum[wave] = incl;
-    __syncthreads();
+    scan(h);
+    if (pass == 0) {
+      const uint32_t above_inf = wave_total();
+      if (above_inf < (uint32_t)need) {            // uniform: all of those are taken, the rest from -inf down
+        uint32_t inf = 0u, low = kNegInfKey;       // low, sh21 opaque: nothing per entry is kept from above
+        int sh21 = 21;
+        asm volatile("" : "+s"(low), "+s"(sh21));
+#pragma unroll
+        for (int j = 0; j < J; ++j) inf += key[j] == low ? 1u : 0u;
+        inf = wave_incl_scan(inf, lane);
+        __syncthreads();                           // wsum read
+        if (lane == 63) sh.wsum[wave] = inf;
+        __syncthreads();
+        if (wave_total() >= (uint32_t)need - above_inf) {   // the k-th best is -inf itself
+          prefix = low;
+          need -= (int)above_inf;
+          __syncthreads();                         // wsum read
+          break;
+        }
+        // the k-th best is a NaN below -inf: count every entry of the row
+        __syncthreads();
+        clear(0);
+        __syncthreads();
+        forget();
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          atomicAdd(&h[p0 + 64 * j < nb ? key[j] >> sh21 : dummy], 1u);
+          if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+        scan(h);
+      }
+    }
     uint32_t above = incl - tot;
 #pragma unroll
     for (int w = 0; w < NW; ++w) above += w < wave ? sh.wsum[w] : 0u;

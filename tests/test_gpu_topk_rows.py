@@ -43,6 +43,22 @@ def test_rows_equal_few_rows(gpu, rows, nb, k, kind):
     assert torch.equal(got, few)
 
 
+@pytest.mark.parametrize("nb,k", [(2048, 600), (10240, 2048), (32768, 512)])
+@pytest.mark.parametrize("inf", [0.0, 0.02, 0.5])
+def test_rows_down_to_infinity_and_below(gpu, nb, k, inf):
+    """The k-th best is -inf, or a NaN below it: entries the first histogram leaves out."""
+    from dsv41 import _abi
+    g = torch.Generator(device="cuda").manual_seed(nb)
+    x = torch.full((512, 1, nb), -float("nan"), device="cuda")
+    x.view(torch.int32).masked_fill_(torch.rand(x.shape, generator=g, device="cuda") < 0.3, -1)
+    x.masked_fill_(torch.rand(x.shape, generator=g, device="cuda") < inf, -float("inf"))
+    x[:, :, 5:20] = 1.0
+    x.view(torch.int32)[100:200, :, 20:] = -0x400000       # rows of equal NaNs
+    got = _abi.topk_select(x, k, nb, 1, 0)
+    few = torch.cat([_abi.topk_select(x[i:i + 31].contiguous(), k, nb, 1, 0) for i in range(0, 512, 31)])
+    assert torch.equal(got, few)
+
+
 def test_rows_of_several_queries(gpu):
     """Visibility follows the query, row % n, also with rows of several sequences and k >= nb."""
     from dsv41 import _abi
