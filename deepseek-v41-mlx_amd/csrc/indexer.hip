@@ -395,6 +395,17 @@ __device__ __forceinline__ f32x4 mfma_mxfp4(uint4 a, int sa, uint4 b, int sb) {
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, f32x4{0.f, 0.f, 0.f, 0.f}, 4, 4, 0, sa, 0, sb);
 }
 
+// mfma_mxfp4 with the query's scale in byte `ht` (a constant after unrolling) of sa.
+__device__ __forceinline__ f32x4 mfma_mxfp4_tile(uint4 a, int sa, int ht, uint4 b, int sb) {
+  const i32x8 av = {(int)a.x, (int)a.y, (int)a.z, (int)a.w, 0, 0, 0, 0};
+  const i32x8 bv = {(int)b.x, (int)b.y, (int)b.z, (int)b.w, 0, 0, 0, 0};
+  const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+  if (ht == 0) return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, z, 4, 4, 0, sa, 0, sb);
+  if (ht == 1) return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, z, 4, 4, 1, sa, 0, sb);
+  if (ht == 2) return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, z, 4, 4, 2, sa, 0, sb);
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, z, 4, 4, 3, sa, 0, sb);
+}
+
 // fp8 keys: an fp4 e2m1 query (A, cbsz = 4) against e4m3 keys (B, blgp = 0). With 8-bit
 // operands the 16x16x128 instruction takes a lane group's 32 bytes as two 16-channel halves:
 // lane group g supplies channels [16g, 16g+16) in bytes 0-15 and [64+16g, 64+16g+16) in bytes
@@ -423,6 +434,8 @@ template <int U, bool KF8> struct MxBatch {
 };
 
 constexpr int kMxThreads = 512;  // 8 waves
+constexpr int kMxChunkThreads = 256;   // indexer_mx_chunk_kernel: 4 waves,
+constexpr int kMxChunkTiles = 8;       // each holding 8 head tiles of queries
 
 // KF8: the keys are fp8 e4m3 rows (128 code bytes) whose ue8m0 scale word (one byte per 32
 // channels) covers 2^ks_shift rows (1 or 32); the query stays MXFP4.
@@ -553,6 +566,112 @@ __global__ __launch_bounds__(kMxThreads) void indexer_score_mx_kernel(
   }
 }
 
+// MXFP4 keys, many queries per batch row: a wave scores NQ consecutive queries against every key
+// batch it loads, so a key row is read from L2 once per NQ queries instead of once per query. The
+// query blocks are small enough to stay in registers (4 code, 1 packed scale and 4 weight registers
+// per head tile and query), so the keys need no LDS and the waves no barriers: the four waves of a
+// workgroup take 64-row blocks of the range in turn, two register batches in flight each. Sums are
+// indexer_score_mx_kernel's, addition for addition; four tiles' head sums are reduced together and
+// leave as one 256-byte store per query. Bound by issue: a 16 x 16 tile of one head tile is one fp4
+// MFMA and 8 VALU instructions (max and fma per product, 32 cycles). 1,999 queries x 16,359 keys,
+// causal: 32 heads 200 us with a workgroup per query (bound by its key loads and 64-byte stores) ->
+// 121 us; 64 heads 188 us, 16 heads 63 us here. NQ * HT = 8 head tiles at three waves per SIMD (168
+// registers); the same at 32 heads with 4 tiles 141 us, 16 tiles 154 us, 8 tiles in 512-thread
+// workgroups of 128 registers 127 us.
+template <int HT, bool CAND>
+__global__ __launch_bounds__(kMxChunkThreads, 3) void indexer_mx_chunk_kernel(
+    const uint8_t* __restrict__ qcodes, const uint8_t* __restrict__ qscales, const bf16_t* __restrict__ w_raw,
+    float w_scale, const uint8_t* __restrict__ kcodes, int64_t kc_bstride, const uint8_t* __restrict__ kscales,
+    int64_t ks_bstride, const uint8_t* __restrict__ cand, float* __restrict__ scores, int n, int nb, int start_pos,
+    int ratio, int rows_per_wg) {
+  constexpr int H = HT * 16, DIM = 128, NQ = kMxChunkTiles / HT, U = 4;
+  constexpr int STRIDE = 16 * U * (kMxChunkThreads / 64);
+  const int groups = (n + NQ - 1) / NQ;
+  const int b = blockIdx.y / groups, s0 = (blockIdx.y - b * groups) * NQ;
+  const int nq = min(NQ, n - s0);
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = blockIdx.x * rows_per_wg, r1 = min(r0 + rows_per_wg, nb);
+  const int vis_end = max(r0, min(r1, (start_pos + s0 + nq) / ratio));   // the group's last query sees most
+  float* out = scores + ((int64_t)b * n + s0) * nb;
+  for (int j = 0; j < nq; ++j)             // rows past the group's visibility
+    for (int t = vis_end + tid; t < r1; t += kMxChunkThreads) out[(int64_t)j * nb + t] = -INFINITY;
+  if (vis_end <= r0) return;               // uniform: nothing visible in this row range
+
+  // uniform bases of the range and 32-bit offsets: 64-bit lane addresses would not fit the registers
+  const int seen_rows = vis_end - r0;
+  const uint8_t* kcb = kcodes + (int64_t)b * kc_bstride + (int64_t)r0 * (DIM / 2);
+  const uint8_t* ksb = kscales + (int64_t)b * ks_bstride + (int64_t)r0 * (DIM / 32);
+  struct Keys {
+    u32x4 k[U];
+    uint32_t sc[U];
+  };
+  auto load = [&](Keys& kk, int t0) {      // t0: rows from the range's first
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t row = (uint32_t)min(t0 + 16 * u + l16, seen_rows - 1);   // clamp: stays inside the cache
+      kk.k[u] = ld_u32x4(kcb + (row * (DIM / 2) + (uint32_t)g * 16u));
+      kk.sc[u] = *reinterpret_cast<const uint32_t*>(ksb + row * (DIM / 32));
+    }
+  };
+  int t0 = 16 * U * wave;
+  Keys ba, bb;
+  load(ba, t0);
+  uint4 qa[NQ][HT];
+  uint32_t qsa[NQ];                        // byte ht: the scale of head tile ht's block g
+  float wv[NQ][HT][4];
+#pragma unroll
+  for (int j = 0; j < NQ; ++j) {           // past the last query: the last one again, not stored
+    const int64_t qi = (int64_t)b * n + s0 + min(j, nq - 1);
+    const bf16_t* wrow = w_raw + qi * H;
+    qsa[j] = 0u;
+#pragma unroll
+    for (int ht = 0; ht < HT; ++ht) {
+      const int64_t hq = qi * H + ht * 16 + l16;
+      qa[j][ht] = *reinterpret_cast<const uint4*>(qcodes + hq * (DIM / 2) + g * 16);
+      qsa[j] |= (uint32_t)qscales[hq * (DIM / 32) + g] << (8 * ht);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wv[j][ht][i] = round_bf16(bf2f(wrow[ht * 16 + 4 * g + i]) * w_scale);
+    }
+  }
+  auto compute = [&](const Keys& kk, int t0) {
+    const int row = t0 + lane;             // the row whose sums this lane stores
+    int sb[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) sb[u] = (int)((kk.sc[u] >> (8 * g)) & 0xFFu);
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+      const int64_t base = ((int64_t)b * n + s0 + min(j, nq - 1)) * nb + r0;
+      uint32_t keep = 1u;
+      if constexpr (CAND) keep = (cand + base)[(uint32_t)min(row, seen_rows - 1)];
+      float part[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        part[u] = 0.0f;
+#pragma unroll
+        for (int ht = 0; ht < HT; ++ht) {
+          const f32x4 acc = mfma_mxfp4_tile(qa[j][ht], (int)qsa[j], ht, as_uint4(kk.k[u]), sb[u]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) part[u] += relu_bits(acc[i]) * wv[j][ht][i];
+        }
+      }
+      const float v = sum_rows4x4(part[0], part[1], part[2], part[3]);
+      const bool seen = r0 + row < (start_pos + s0 + j + 1) / ratio && keep != 0u;
+      if (j < nq && row < seen_rows) (scores + base)[(uint32_t)row] = seen ? v : -INFINITY;
+      __builtin_amdgcn_sched_barrier(0);   // one query's products at a time
+    }
+  };
+  while (t0 < seen_rows) {                 // wave-uniform
+    load(bb, t0 + STRIDE);
+    compute(ba, t0);
+    t0 += STRIDE;
+    if (t0 >= seen_rows) break;
+    load(ba, t0 + STRIDE);
+    compute(bb, t0);
+    t0 += STRIDE;
+  }
+}
+
 // Prefill (many queries per batch row): a workgroup scores 8 consecutive queries of one batch row
 // -- one per wave -- against a range of at most kPfRows keys. The keys stream
 // through an LDS ring in 64-row chunks with global_load_lds, so each key row is read from HBM
@@ -568,7 +687,7 @@ __global__ __launch_bounds__(kMxThreads) void indexer_score_mx_kernel(
 // 16-row tile none of whose rows is a visible candidate of the query is not multiplied. Masked
 // chunks used to run on the decode kernel, one workgroup per query and row range, which reads every
 // key again for every query: 2,048 queries x 32,768 keys, 32 heads, half of the entries kept,
-// 1,181 us there with the selection fused against 387 us here (+ 297 us for the selection).
+// 1,181 us there with the selection fused against 387 us here (+ 86 us for the selection).
 constexpr int kPfThreads = 512;        // 8 waves = 8 queries
 constexpr int kPfChunk = 64;           // key rows per ring slot (16 KB at 128 channels)
 constexpr int kPfSlots = 3;            // ring slots: 2 chunks in flight (48 KB: two workgroups per CU)
@@ -975,6 +1094,22 @@ static int mx_score_entry(const char* what, bool kf8, const uint8_t* q_codes, co
   DSV41_REQUIRE(kc_bstride % 16 == 0 && ks_bstride % 4 == 0, DSV41_E_ARG,
                 "%s: kc_bstride must be a multiple of 16 bytes, ks_bstride of 4", what);
   if ((int64_t)bsz * n == 0 || nb == 0) return 0;
+  if (!kf8 && n >= 8 && (heads == 64 || heads == 32 || heads == 16)) {
+    const int nq = kMxChunkTiles * 16 / heads;
+    const int64_t groups = (int64_t)bsz * ((n + nq - 1) / nq);
+    const int rows = prefill_rows(groups, nb);
+    const dim3 cgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
+#define DSV41_MXCHUNK_CASE(HT_, CAND_)                                                                        \
+    if (heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                              \
+      hipLaunchKernelGGL((indexer_mx_chunk_kernel<HT_, CAND_>), cgrid, dim3(kMxChunkThreads), 0, stream, q_codes, \
+                         q_scales, (const bf16_t*)w_raw, w_scale, k_codes, kc_bstride, k_scales, ks_bstride,  \
+                         candidates, scores, n, nb, start_pos, ratio, rows);                                  \
+      return check_launch(what);                                                                              \
+    }
+    DSV41_MXCHUNK_CASE(4, false) DSV41_MXCHUNK_CASE(2, false) DSV41_MXCHUNK_CASE(1, false)
+    DSV41_MXCHUNK_CASE(4, true) DSV41_MXCHUNK_CASE(2, true) DSV41_MXCHUNK_CASE(1, true)
+#undef DSV41_MXCHUNK_CASE
+  }
   int rows_per_wg = 0;
   const dim3 grid = idx_grid((int64_t)nb * bsz * n, nb, bsz * n, &rows_per_wg);
   const int shift = ks_rb == 32 ? 5 : 0;

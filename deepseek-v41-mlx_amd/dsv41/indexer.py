@@ -42,12 +42,13 @@ def select_candidate_blocks(scores: torch.Tensor, lens, topk_blocks: int,
                                  _lens_tensor(lens, scores.device))
 
 
-# Queries per sequence from which bf16 keys take the scoring and the selection as two calls: the
-# scoring kernel then reads each key once per 8 queries, where the fused form's reads every key for
-# every query. Only masked layers meet the choice (without a mask the fused form stops at 8 queries
-# anyway). 32 heads, fused against score + select: 8 queries x 65,536 keys 42.9 against 30.1 us,
-# 64 x 8,192 22.0 against 21.7 us, 2,048 x 32,768 1,181 against 684 us; no size measured from 8
-# queries on favoured the fused form.
+# Queries per sequence from which bf16 and MXFP4 keys take the scoring and the selection as two calls:
+# the scoring kernel then reads each key once per several queries, where the fused form's reads every
+# key for every query. Only masked layers meet the choice (without a mask the fused form stops at 8
+# queries anyway). 32 heads, fused against score + select: bf16 keys 8 queries x 65,536 keys 42.9
+# against 30.1 us, 64 x 8,192 22.0 against 21.7 us, 2,048 x 32,768 1,181 against 470 us; MXFP4 keys
+# 8 x 65,536 38.0 against 27.5 us, 64 x 8,192 21.8 against 21.3 us, 2,048 x 32,768 655 against 351 us;
+# no size measured from 8 queries on favoured the fused form.
 CHUNK_QUERIES = 8
 
 
@@ -135,7 +136,7 @@ class Indexer(torch.nn.Module):
                 raise ValueError("an MXFP4 index cache holds fp4 fake-quantized keys; QAT is disabled")
             q_mx = _abi.index_q_prep_mxfp4(q, cos, sin, rd, start_pos)
             nb = index_k.codes.shape[1]
-            if not self.is_candidate_source:
+            if not self.is_candidate_source and n < CHUNK_QUERIES:
                 idx = _abi.indexer_topk_mxfp4(q_mx, w_raw, w_scale, index_k.codes, index_k.scales, nb, start_pos,
                                               self.ratio, self.index_topk, offset, cand)
                 if idx is not None:

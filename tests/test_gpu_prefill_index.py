@@ -68,3 +68,33 @@ def test_masked_selection_same_in_both_forms(gpu, n, nb):
     two = _abi.topk_select(_abi.indexer_score(q, w, 0.07, k, nb - n, 1, cand), 128, nb - n, 1, 7)
     fused = _abi.indexer_topk(q, w, 0.07, k, nb - n, 1, 128, 7, cand)
     assert fused is not None and torch.equal(two, fused)
+
+
+@pytest.mark.parametrize("b,n,heads,nb,start,ratio,keep", [
+    (1, 8, 32, 1, 0, 1, None),           # one key; a query before it
+    (2, 9, 64, 63, 40, 1, 0.5),          # partial query group, partial key block, causal edge inside it
+    (1, 17, 16, 513, 700, 1, None),      # the range's waves get uneven shares
+    (3, 11, 32, 2049, 2040, 1, 0.3),     # a last range of one key
+    (1, 64, 32, 4101, 16388, 4, None),   # several ranges, queries before and after the last key
+    (2, 13, 64, 1024, 4084, 4, 0.05),
+])
+def test_mxfp4_chunk_scores_equal_per_query(gpu, b, n, heads, nb, start, ratio, keep):
+    from dsv41 import _abi
+    g = torch.Generator(device="cuda").manual_seed(nb + n)
+
+    def ints(lo, hi, *shape):
+        return torch.randint(lo, hi, shape, generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+
+    qc, qs = ints(0, 256, b, n, heads, 64), ints(118, 132, b, n, heads, 4)
+    kc, ks = ints(0, 256, b, nb + 5, 64), ints(118, 132, b, nb + 5, 4)      # a longer cache
+    w = torch.randn(b, n, heads, generator=g, device="cuda").bfloat16()
+    cand = None
+    if keep is not None:
+        cand = torch.rand(b, n, nb, generator=g, device="cuda").lt(keep).to(torch.uint8).mul_(7).contiguous()
+    got = _abi.indexer_score_mxfp4((qc, qs), w, 0.07, kc, ks, nb, start, ratio, cand)
+    rows = []
+    for s in range(n):                   # each query by a call of its own: the one-query kernel
+        c = None if cand is None else cand[:, s:s + 1].contiguous()
+        rows.append(_abi.indexer_score_mxfp4((qc[:, s:s + 1].contiguous(), qs[:, s:s + 1].contiguous()),
+                                             w[:, s:s + 1].contiguous(), 0.07, kc, ks, nb, start + s, ratio, c))
+    assert torch.equal(got, torch.cat(rows, 1))
