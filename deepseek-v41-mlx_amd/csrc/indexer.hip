@@ -688,9 +688,9 @@ __global__ __launch_bounds__(kMxChunkThreads, 3) void indexer_mx_chunk_kernel(
 // chunks used to run on the decode kernel, one workgroup per query and row range, which reads every
 // key again for every query: 2,048 queries x 32,768 keys, 32 heads, half of the entries kept,
 // 1,181 us there with the selection fused against 387 us here (+ 86 us for the selection).
-constexpr int kPfThreads = 512;        // 8 waves = 8 queries
+constexpr int kPfQueries = 8;          // queries per workgroup
 constexpr int kPfChunk = 64;           // key rows per ring slot (16 KB at 128 channels)
-constexpr int kPfSlots = 3;            // ring slots: 2 chunks in flight (48 KB: two workgroups per CU)
+constexpr int kPfSlots = 3;            // ring slots of bf16 keys: 2 chunks in flight (48 KB)
 constexpr int kPfRows = 2048;          // most key rows per workgroup
 
 // One bit per byte of v: bit i set where byte i is not 0.
@@ -699,49 +699,66 @@ __device__ __forceinline__ uint32_t nonzero_bytes(uint32_t v) {
   return ((t >> 7) * 0x10204080u) >> 28;   // bits 0, 8, 16, 24 -> 28, 29, 30, 31 (no two products overlap)
 }
 
-// (__launch_bounds__'s second argument, 4 waves per SIMD, caps VGPRs at 128 so that two
-// workgroups share a CU)
-template <int HT, bool CAND>
-__global__ __launch_bounds__(kPfThreads, 4) void indexer_prefill_kernel(
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ w_raw, float w_scale, const bf16_t* __restrict__ kcache,
-    int64_t k_bstride, const uint8_t* __restrict__ cand, float* __restrict__ scores, int n, int nb, int start_pos,
-    int ratio, int rows_per_wg, int cand_vec) {
-  constexpr int H = HT * 16, DIM = 128, KS = 4;
-  constexpr int ROWB = DIM * 2;                          // 256 bytes per key row
+// NQ queries per wave, 8 per workgroup. NQ = 1: 8 waves, 4 per SIMD (128 registers, two workgroups
+// share a CU). NQ = 2 (16 and 32 heads, no mask): 4 waves, 3 per SIMD (168 registers, three
+// workgroups), each key operand read from LDS once for two queries; one per wave, the 32-head LDS
+// reads take as long as the MFMAs. 4,096 queries x 36,864 keys, 32 heads 993 -> 926 us, 2,048 x 8,192
+// 116 -> 111 us, 16 heads 78 -> 74 us. Under a mask two queries share few empty tiles: 32 heads,
+// 2,048 x 32,768, half kept 385 us with one, 402 us with two.
+//
+// F8: e4m3 keys with ue8m0 scales, dequantized once per workgroup on their way into the ring (exact
+// in bf16, indexer_decode_kernel's operands bit for bit), through registers one chunk ahead instead of
+// the LDS copies. They ran a workgroup per query on indexer_decode_kernel: 2,048 queries x 8,192 keys,
+// 32 heads 199 -> 115 us, 64 heads 280 -> 213 us; masked 2,048 x 32,768 845 -> 388 us.
+template <int HT, int NQ, bool CAND, bool F8>
+__global__ __launch_bounds__(64 * kPfQueries / NQ, NQ == 1 ? 4 : 3) void indexer_prefill_kernel(
+    const bf16_t* __restrict__ q, const bf16_t* __restrict__ w_raw, float w_scale, const void* __restrict__ kcache,
+    int64_t k_bstride, const uint8_t* __restrict__ kscale, int64_t ks_bstride, int ks_shift,
+    const uint8_t* __restrict__ cand, float* __restrict__ scores, int n, int nb, int start_pos, int ratio,
+    int rows_per_wg, int cand_vec) {
+  constexpr int H = HT * 16, DIM = 128, KS = 4, NW = kPfQueries / NQ, NT = 64 * NW;
+  constexpr int ROWB = DIM * 2;                          // 256 bytes per staged key row
   constexpr int CHUNKB = kPfChunk * ROWB;
-  constexpr int NL = CHUNKB / 1024 / (kPfThreads / 64);  // copies per wave per chunk
-  static_assert(NL * 1024 * (kPfThreads / 64) == CHUNKB, "a chunk splits evenly into 1 KB copies per wave");
-  __shared__ __align__(16) uint8_t ring[kPfSlots * CHUNKB];
-  __shared__ __align__(8) uint32_t cbits[CAND ? kPfThreads / 64 : 1][CAND ? kPfRows / 32 : 2];
+  constexpr int SLOTS = F8 ? 2 : kPfSlots;
+  constexpr int NL = CHUNKB / 1024 / NW;                 // bf16 keys: copies per wave per chunk
+  constexpr int NP = kPfChunk * DIM / 16 / NT;           // fp8 keys: 16-byte pieces per thread per chunk
+  static_assert(NL * 1024 * NW == CHUNKB && NP * 16 * NT == kPfChunk * DIM, "chunks split evenly over the waves");
+  __shared__ __align__(16) uint8_t ring[SLOTS * CHUNKB];
+  __shared__ __align__(8) uint32_t cbits[CAND ? kPfQueries : 1][CAND ? kPfRows / 32 : 2];
 
-  const int groups = (n + 7) / 8;
+  const int groups = (n + kPfQueries - 1) / kPfQueries;
   const int b = blockIdx.y / groups, sg = blockIdx.y - (blockIdx.y / groups) * groups;
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int s = sg * 8 + wave;
-  const bool qok = s < n;
-  const int s_last = min(sg * 8 + 7, n - 1);
+  const int s0 = sg * kPfQueries + wave * NQ;            // this wave's first query
+  const int s_last = min(sg * kPfQueries + kPfQueries - 1, n - 1);
   const int lens_max = (start_pos + s_last + 1) / ratio;
-  const int lens = (start_pos + min(s, n - 1) + 1) / ratio;
   const int r0 = blockIdx.x * rows_per_wg, r1 = min(r0 + rows_per_wg, nb);
   const int vis_end = max(r0, min(r1, lens_max));
-  float* out = scores + ((int64_t)b * n + min(s, n - 1)) * nb;
+  float* out[NQ];
+  int lens[NQ];
+#pragma unroll
+  for (int j = 0; j < NQ; ++j) {
+    const int sq = min(s0 + j, n - 1);
+    out[j] = scores + ((int64_t)b * n + sq) * nb;
+    lens[j] = (start_pos + sq + 1) / ratio;
+  }
   // rows past the group's visibility: -inf for each of its queries
   {
     const int span = r1 - vis_end;
-    for (int e = tid; e < 8 * span; e += kPfThreads) {
+    for (int e = tid; e < kPfQueries * span; e += NT) {
       const int qq = e / span, row = vis_end + (e - qq * span);
-      if (sg * 8 + qq < n) scores[((int64_t)b * n + sg * 8 + qq) * nb + row] = -INFINITY;
+      if (sg * kPfQueries + qq < n) scores[((int64_t)b * n + sg * kPfQueries + qq) * nb + row] = -INFINITY;
     }
   }
   if (vis_end <= r0) return;               // uniform: nothing visible in this row range
   const int nchunks = (vis_end - r0 + kPfChunk - 1) / kPfChunk;
-  const uint8_t* kb = reinterpret_cast<const uint8_t*>(kcache + (int64_t)b * k_bstride);
+  const uint8_t* kb = reinterpret_cast<const uint8_t*>(kcache) + (int64_t)b * k_bstride * (F8 ? 1 : 2);
   const uint32_t ring_base = lds_offset(ring);
-  // chunk c -> slot c % kPfSlots; copy i (1 KB = 4 rows) goes to wave i / NL. Lane l of a copy
+  // bf16: chunk c -> slot c % SLOTS; copy i (1 KB = 4 rows) goes to wave i / NL. Lane l of a copy
   // lands at row 4i + l/16, position l%16, and so loads column chunk (l%16) ^ (row % 16).
   auto issue = [&](int c) {
-    const int slot = c % kPfSlots;
+    const int slot = c % SLOTS;
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
       const int ins = wave * NL + j;
@@ -752,97 +769,164 @@ __global__ __launch_bounds__(kPfThreads, 4) void indexer_prefill_kernel(
       dma16_vaddr(reinterpret_cast<uint64_t>(kb + (int64_t)row * ROWB + col * 16), dst);
     }
   };
-  issue(0);
-  // the query's A operands and head weights (an idle wave takes the last query and stores nothing)
-  const int64_t qi = (int64_t)b * n + min(s, n - 1);
-  bf16x8 qa[HT][KS];
-  float wv[HT][4];
-  {
+  // fp8: piece tid + NT i of a chunk is 16 channels of row piece / 8, loaded one chunk ahead into
+  // registers with the row's scale word and written as bf16 at the same swizzled place
+  u32x4 raw[F8 ? NP : 1];
+  uint32_t rsc[F8 ? NP : 1];
+  const uint8_t* sbase = kscale + (int64_t)b * ks_bstride;
+  auto load8 = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int pc = tid + NT * i;
+      const int row = min(r0 + c * kPfChunk + (pc >> 3), vis_end - 1);
+      raw[i] = ld_u32x4(kb + (int64_t)row * DIM + (pc & 7) * 16);
+      rsc[i] = *reinterpret_cast<const uint32_t*>(sbase + (int64_t)(row >> ks_shift) * (DIM / 32));
+    }
+  };
+  auto store8 = [&](int c) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int pc = tid + NT * i, rloc = pc >> 3, c16 = pc & 7;
+      const float sc = e8m0_to_float((rsc[i] >> (8 * (c16 >> 1))) & 255u);
+      uint8_t* rowp = ring + (c % SLOTS) * CHUNKB + rloc * ROWB;
+      *reinterpret_cast<bf16x8*>(rowp + (((2 * c16) ^ (rloc & 15)) * 16)) = dequant_e4m3x8(raw[i][0], raw[i][1], sc);
+      *reinterpret_cast<bf16x8*>(rowp + (((2 * c16 + 1) ^ (rloc & 15)) * 16)) = dequant_e4m3x8(raw[i][2], raw[i][3], sc);
+    }
+  };
+  if constexpr (F8) load8(0);
+  else issue(0);
+  // the queries' A operands and head weights (past the last query: the last one again, not stored)
+  bf16x8 qa[NQ][HT][KS];
+  float wv[NQ][HT][4];
+#pragma unroll
+  for (int j = 0; j < NQ; ++j) {
+    const int64_t qi = (int64_t)b * n + min(s0 + j, n - 1);
     const bf16_t* qrow = q + qi * H * DIM;
-#pragma unroll
-    for (int ht = 0; ht < HT; ++ht)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) qa[ht][ks] = ld_bf16x8(qrow + (ht * 16 + l16) * DIM + ks * 32 + g * 8);
     const bf16_t* wrow = w_raw + qi * H;
 #pragma unroll
-    for (int ht = 0; ht < HT; ++ht)
+    for (int ht = 0; ht < HT; ++ht) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) wv[ht][i] = round_bf16(bf2f(wrow[ht * 16 + 4 * g + i]) * w_scale);
+      for (int ks = 0; ks < KS; ++ks) qa[j][ht][ks] = ld_bf16x8(qrow + (ht * 16 + l16) * DIM + ks * 32 + g * 8);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wv[j][ht][i] = round_bf16(bf2f(wrow[ht * 16 + 4 * g + i]) * w_scale);
+    }
   }
   if constexpr (CAND) {                    // this wave's mask bits: lane l holds rows r0 + 32 l .. + 31
-    const uint8_t* cr = cand + qi * nb + r0;
-    const int left = min(r1, lens) - r0;   // bytes past the range or the query's visibility stay 0
-    uint32_t bits = 0u;
-    if (cand_vec) {                        // rows of the mask 16-byte aligned (nb a multiple of 16)
+    for (int j = 0; j < NQ; ++j) {
+      const int sq = min(s0 + j, n - 1);
+      const uint8_t* cr = cand + ((int64_t)b * n + sq) * nb + r0;
+      const int left = min(r1, lens[j]) - r0;   // bytes past the range or the query's visibility stay 0
+      uint32_t bits = 0u;
+      if (cand_vec) {                      // rows of the mask 16-byte aligned (nb a multiple of 16)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (32 * lane + 16 * h < left) {
-          const uint4 m = *reinterpret_cast<const uint4*>(cr + 32 * lane + 16 * h);
-          bits |= (nonzero_bytes(m.x) | nonzero_bytes(m.y) << 4 | nonzero_bytes(m.z) << 8 | nonzero_bytes(m.w) << 12)
-                  << (16 * h);
+        for (int h = 0; h < 2; ++h) {
+          if (32 * lane + 16 * h < left) {
+            const uint4 m = *reinterpret_cast<const uint4*>(cr + 32 * lane + 16 * h);
+            bits |= (nonzero_bytes(m.x) | nonzero_bytes(m.y) << 4 | nonzero_bytes(m.z) << 8 | nonzero_bytes(m.w) << 12)
+                    << (16 * h);
+          }
+        }
+        const int keep = left - 32 * lane; // the last piece may reach past the query's visibility
+        if (keep < 32) bits &= keep > 0 ? (1u << keep) - 1u : 0u;
+      } else {                             // 64 bytes per load, packed by a ballot
+#pragma unroll 8
+        for (int i = 0; i < kPfRows / 64; ++i) {
+          const int t = 64 * i + lane;
+          const uint64_t m = __ballot(t < left && cr[min(t, max(left - 1, 0))] != 0);
+          bits = lane == 2 * i ? (uint32_t)m : (lane == 2 * i + 1 ? (uint32_t)(m >> 32) : bits);
         }
       }
-      const int keep = left - 32 * lane;   // the last piece may reach past the query's visibility
-      if (keep < 32) bits &= keep > 0 ? (1u << keep) - 1u : 0u;
-    } else {                               // 64 bytes per load, packed by a ballot
-#pragma unroll 8
-      for (int j = 0; j < kPfRows / 64; ++j) {
-        const int t = 64 * j + lane;
-        const uint64_t m = __ballot(t < left && cr[min(t, max(left - 1, 0))] != 0);
-        bits = lane == 2 * j ? (uint32_t)m : (lane == 2 * j + 1 ? (uint32_t)(m >> 32) : bits);
-      }
+      cbits[wave * NQ + j][lane] = bits;   // read back by this wave only
     }
-    cbits[wave][lane] = bits;              // read back by this wave only
   }
-  // query, weights and chunk 0 complete (a wait the compiler sees: no drain inside the loop)
-  __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
-  for (int c = 1; c < nchunks && c < kPfSlots - 1; ++c) issue(c);
+  if constexpr (F8) {
+    store8(0);
+    if (nchunks > 1) load8(1);
+  } else {
+    // queries, weights and chunk 0 complete (a wait the compiler sees: no drain inside the loop)
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
+    for (int c = 1; c < nchunks && c < SLOTS - 1; ++c) issue(c);
+  }
 
   for (int c = 0; c < nchunks; ++c) {
-    const int after = min(nchunks - 1 - c, kPfSlots - 2);   // younger chunks allowed in flight
-    static_assert(kPfSlots <= 4, "waits below cover at most 2 younger chunks");
-    if (after >= 2) wait_vmcnt<2 * NL>();
-    else if (after == 1) wait_vmcnt<NL>();
-    else wait_vmcnt<0>();
+    if constexpr (!F8) {
+      const int after = min(nchunks - 1 - c, SLOTS - 2);    // younger chunks allowed in flight
+      static_assert(F8 || SLOTS <= 4, "waits below cover at most 2 younger chunks");
+      if (after >= 2) wait_vmcnt<2 * NL>();
+      else if (after == 1) wait_vmcnt<NL>();
+      else wait_vmcnt<0>();
+    }
     __syncthreads();                       // chunk c landed for every wave; chunk c-1 consumed
-    if (c + kPfSlots - 1 < nchunks) issue(c + kPfSlots - 1);
-    const uint8_t* buf = ring + (c % kPfSlots) * CHUNKB;
-    float part[4];                         // this lane's head group's share of the chunk's four 16-row tiles
+    if constexpr (F8) {
+      if (c + 1 < nchunks) store8(c + 1);
+      if (c + 2 < nchunks) load8(c + 2);
+    } else {
+      if (c + SLOTS - 1 < nchunks) issue(c + SLOTS - 1);
+    }
+    const uint8_t* buf = ring + (c % SLOTS) * CHUNKB;
+    float part[NQ][4];                     // this lane's head group's share of the chunk's four 16-row tiles
     static_assert(kPfChunk == 64, "four 16-row tiles per chunk, one row per lane");
-    uint32_t mlo = 0u, mhi = 0u;           // the chunk's mask bits (CAND)
+    uint32_t mlo[NQ], mhi[NQ];             // the chunk's mask bits (CAND)
     if constexpr (CAND) {
-      const uint2 m = *reinterpret_cast<const uint2*>(&cbits[wave][2 * c]);
-      mlo = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.x);
-      mhi = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.y);
+#pragma unroll
+      for (int j = 0; j < NQ; ++j) {
+        const uint2 m = *reinterpret_cast<const uint2*>(&cbits[wave * NQ + j][2 * c]);
+        mlo[j] = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.x);
+        mhi[j] = (uint32_t)__builtin_amdgcn_readfirstlane((int)m.y);
+      }
     }
 #pragma unroll
     for (int kt = 0; kt < 4; ++kt) {
-      part[kt] = 0.0f;
-      if constexpr (CAND)                  // wave-uniform
-        if ((((kt < 2 ? mlo : mhi) >> (16 * (kt & 1))) & 0xFFFFu) == 0u) continue;
-      f32x4 acc[HT];
+      bool any = !CAND;
 #pragma unroll
-      for (int ht = 0; ht < HT; ++ht) acc[ht] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int j = 0; j < NQ; ++j) {
+        part[j][kt] = 0.0f;
+        if constexpr (CAND)                // wave-uniform
+          any = any || (((kt < 2 ? mlo[j] : mhi[j]) >> (16 * (kt & 1))) & 0xFFFFu) != 0u;
+      }
+      if (!any) continue;
       const uint8_t* rowp = buf + (kt * 16 + l16) * ROWB;
+      f32x4 acc[NQ][HT];
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const bf16x8 kop = ld_bf16x8(rowp + (((ks * 4 + g) ^ l16) * 16));
+      for (int j = 0; j < NQ; ++j)
 #pragma unroll
-        for (int ht = 0; ht < HT; ++ht) acc[ht] = mfma16x16x32(qa[ht][ks], kop, acc[ht]);
+        for (int ht = 0; ht < HT; ++ht) acc[j][ht] = f32x4{0.f, 0.f, 0.f, 0.f};
+      bf16x8 kop[KS];
+      auto read = [&](int ks) { kop[ks] = ld_bf16x8(rowp + (((ks * 4 + g) ^ l16) * 16)); };
+      constexpr bool kAhead = !(F8 && HT == 4);    // that instance has no registers for all four reads
+      if constexpr (kAhead) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) read(ks);
+        // behind a tile's branch the scheduler keeps two of the four reads back otherwise (5 % of the
+        // masked kernel at 32 heads)
+        if constexpr (CAND) __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
-      for (int ht = 0; ht < HT; ++ht)
+      for (int ks = 0; ks < KS; ++ks) {
+        if constexpr (!kAhead) read(ks);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) part[kt] += relu_bits(acc[ht][i]) * wv[ht][i];
+        for (int j = 0; j < NQ; ++j)
+#pragma unroll
+          for (int ht = 0; ht < HT; ++ht) acc[j][ht] = mfma16x16x32(qa[j][ht][ks], kop[ks], acc[j][ht]);
+      }
+#pragma unroll
+      for (int j = 0; j < NQ; ++j)
+#pragma unroll
+        for (int ht = 0; ht < HT; ++ht)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) part[j][kt] += relu_bits(acc[j][ht][i]) * wv[j][ht][i];
     }
-    // lane = row of the chunk (row group g holds tile g's sums): one 256-byte store per wave. Summing
+    // lane = row of the chunk (row group g holds tile g's sums): one 256-byte store per query. Summing
     // and storing tile by tile (8 permutes and 8 additions more, four 64-byte stores): 8,192 queries x
     // 10,240 keys x 64 heads 945 us, 911 us this way, in turn.
-    const float v = sum_rows4x4(part[0], part[1], part[2], part[3]);
     const int row = r0 + c * kPfChunk + lane;
-    bool seen = row < lens;
-    if constexpr (CAND) seen = (((lane < 32 ? mlo : mhi) >> (lane & 31)) & 1u) != 0u;
-    if (qok && row < vis_end) out[row] = seen ? v : -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NQ; ++j) {
+      const float v = sum_rows4x4(part[j][0], part[j][1], part[j][2], part[j][3]);
+      bool seen = row < lens[j];
+      if constexpr (CAND) seen = (((lane < 32 ? mlo[j] : mhi[j]) >> (lane & 31)) & 1u) != 0u;
+      if (s0 + j < n && row < vis_end) out[j][row] = seen ? v : -INFINITY;
+    }
   }
 }
 
@@ -944,19 +1028,19 @@ extern "C" int dsv41_indexer_score(const void* q, const void* w_raw, float w_sca
   DSV41_REQUIRE(k_bstride % 8 == 0, DSV41_E_ARG, "%s: k_bstride must be a multiple of 8", what);
   if (n >= 8 && dim == 128 && (heads == 64 || heads == 32 || heads == 16) &&
       (int64_t)bsz * ((n + 7) / 8) < 65536) {
-    const int64_t groups = (int64_t)bsz * ((n + 7) / 8);
+    const int64_t groups = (int64_t)bsz * ((n + kPfQueries - 1) / kPfQueries);
     const int rows = prefill_rows(groups, nb);
     const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
     const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
-#define DSV41_PF_CASE(HT_, CAND_)                                                                           \
+#define DSV41_PF_CASE(HT_, NQ_, CAND_)                                                                      \
     if (heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                             \
-      hipLaunchKernelGGL((indexer_prefill_kernel<HT_, CAND_>), pgrid, dim3(kPfThreads), 0, stream,           \
-                         (const bf16_t*)q, (const bf16_t*)w_raw, w_scale, (const bf16_t*)index_k, k_bstride,   \
-                         candidates, scores, n, nb, start_pos, ratio, rows, cvec);                           \
+      hipLaunchKernelGGL((indexer_prefill_kernel<HT_, NQ_, CAND_, false>), pgrid, dim3(64 * kPfQueries / NQ_), 0, \
+                         stream, (const bf16_t*)q, (const bf16_t*)w_raw, w_scale, index_k, k_bstride, nullptr, \
+                         0, 0, candidates, scores, n, nb, start_pos, ratio, rows, cvec);                      \
       return check_launch(what);                                                                             \
     }
-    DSV41_PF_CASE(4, false) DSV41_PF_CASE(2, false) DSV41_PF_CASE(1, false)
-    DSV41_PF_CASE(4, true) DSV41_PF_CASE(2, true) DSV41_PF_CASE(1, true)
+    DSV41_PF_CASE(4, 1, false) DSV41_PF_CASE(2, 2, false) DSV41_PF_CASE(1, 2, false)
+    DSV41_PF_CASE(4, 1, true) DSV41_PF_CASE(2, 1, true) DSV41_PF_CASE(1, 1, true)
 #undef DSV41_PF_CASE
   }
   int rows_per_wg = 0;
@@ -1040,6 +1124,22 @@ extern "C" int dsv41_indexer_score_fp8(const void* q, const void* w_raw, float w
   DSV41_REQUIRE(k_bstride % 16 == 0 && ks_bstride % 4 == 0, DSV41_E_ARG,
                 "%s: k_bstride must be a multiple of 16 bytes, ks_bstride of 4", what);
   if ((int64_t)bsz * n == 0 || nb == 0) return 0;
+  if (n >= 8 && (heads == 64 || heads == 32 || heads == 16)) {
+    const int64_t groups = (int64_t)bsz * ((n + kPfQueries - 1) / kPfQueries);
+    const int rows = prefill_rows(groups, nb);
+    const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
+    const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
+#define DSV41_PF8_CASE(HT_, NQ_, CAND_)                                                                       \
+    if (heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                              \
+      hipLaunchKernelGGL((indexer_prefill_kernel<HT_, NQ_, CAND_, true>), pgrid, dim3(64 * kPfQueries / NQ_), 0, \
+                         stream, (const bf16_t*)q, (const bf16_t*)w_raw, w_scale, index_k, k_bstride, k_scale, \
+                         ks_bstride, ks_rb == 32 ? 5 : 0, candidates, scores, n, nb, start_pos, ratio, rows, cvec); \
+      return check_launch(what);                                                                              \
+    }
+    DSV41_PF8_CASE(4, 1, false) DSV41_PF8_CASE(2, 2, false) DSV41_PF8_CASE(1, 2, false)
+    DSV41_PF8_CASE(4, 1, true) DSV41_PF8_CASE(2, 1, true) DSV41_PF8_CASE(1, 1, true)
+#undef DSV41_PF8_CASE
+  }
   int rows_per_wg = 0;
   const dim3 grid = idx_grid((int64_t)nb * bsz * n, nb, bsz * n, &rows_per_wg);
   if ((heads == 64 || heads == 32 || heads == 16) && aligned16(w_raw) && aligned16(k_scale) &&

@@ -50,6 +50,11 @@ def select_candidate_blocks(scores: torch.Tensor, lens, topk_blocks: int,
 # 8 x 65,536 38.0 against 27.5 us, 64 x 8,192 21.8 against 21.3 us, 2,048 x 32,768 655 against 351 us;
 # no size measured from 8 queries on favoured the fused form.
 CHUNK_QUERIES = 8
+# The same choice over fp8 keys, whose fused form wins on small chunks (fused against two calls, 9 x 8,192
+# keys, 64 heads 17.7 against 26.1 us, 64 x 2,048 17.4 against 22.7 us) and loses from half a million
+# scores on (64 x 8,192, 32 heads 26.4 against 23.4 us, 8 x 65,536 43.8 against 30.0 us, 2,048 x 32,768
+# 1,048 against 475 us).
+CHUNK_SCORES_FP8 = 1 << 19
 
 
 def weight_scale(n_heads: int, head_dim: int, dtype) -> float:
@@ -149,7 +154,8 @@ class Indexer(torch.nn.Module):
             else:
                 _abi.index_q_prep(q, cos, sin, rd, start_pos)
             nb = index_k.codes.shape[1]
-            if not self.is_candidate_source and q.dtype == torch.bfloat16:
+            if (not self.is_candidate_source and q.dtype == torch.bfloat16
+                    and (n < CHUNK_QUERIES or bsz * n * nb < CHUNK_SCORES_FP8)):
                 idx = _abi.indexer_topk_fp8(q, w_raw, w_scale, index_k.codes, index_k.scales, index_k.rb, nb, start_pos,
                                             self.ratio, self.index_topk, offset, cand)
                 if idx is not None:

@@ -98,3 +98,29 @@ def test_mxfp4_chunk_scores_equal_per_query(gpu, b, n, heads, nb, start, ratio, 
         rows.append(_abi.indexer_score_mxfp4((qc[:, s:s + 1].contiguous(), qs[:, s:s + 1].contiguous()),
                                              w[:, s:s + 1].contiguous(), 0.07, kc, ks, nb, start + s, ratio, c))
     assert torch.equal(got, torch.cat(rows, 1))
+
+
+@pytest.mark.parametrize("b,n,heads,nb,start,ratio,rb,keep", [
+    (1, 8, 32, 1, 0, 1, 32, None),       # one key; a query before it
+    (2, 9, 64, 63, 40, 1, 1, 0.5),       # partial query group, partial key chunk, causal edge inside it
+    (1, 17, 16, 513, 700, 1, 32, 0.02),  # most 16-row tiles empty
+    (3, 11, 32, 2049, 2040, 1, 1, 0.3),  # a last range of one key
+    (1, 64, 32, 4101, 16388, 4, 32, None),
+    (2, 13, 64, 1024, 4084, 4, 32, None),
+])
+def test_fp8_chunk_scores_equal_per_query(gpu, b, n, heads, nb, start, ratio, rb, keep):
+    from dsv41 import _abi
+    g, q, w, k = _inputs(b, n, heads, nb, nb + n, spare=5)
+    codes = k.to(torch.float8_e4m3fn).view(torch.uint8)
+    scales = torch.randint(118, 132, (b, (nb + 5 + rb - 1) // rb, 4), generator=g, device="cuda", dtype=torch.int32)
+    scales = scales.to(torch.uint8)
+    cand = None
+    if keep is not None:
+        cand = torch.rand(b, n, nb, generator=g, device="cuda").lt(keep).to(torch.uint8).contiguous()
+    got = _abi.indexer_score_fp8(q, w, 0.07, codes, scales, rb, nb, start, ratio, cand)
+    rows = []
+    for s in range(n):                   # each query by a call of its own: the one-query kernel
+        c = None if cand is None else cand[:, s:s + 1].contiguous()
+        rows.append(_abi.indexer_score_fp8(q[:, s:s + 1].contiguous(), w[:, s:s + 1].contiguous(), 0.07, codes, scales,
+                                           rb, nb, start + s, ratio, c))
+    assert torch.equal(got, torch.cat(rows, 1))
