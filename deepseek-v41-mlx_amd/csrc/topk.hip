@@ -256,26 +256,63 @@ struct StripeShared {
   uint32_t pick[3];
 };
 
-constexpr uint32_t kNegInfKey = 0x007FFFFFu;     // order_key(-INFINITY)
+constexpr uint32_t kNegInfKey = 0x007FFFFFu, kInfKey = 0xFF800000u;   // order_key of -INFINITY, INFINITY
 
-// LISTS: stage 1 of the two-stage selection (below) over `chunks` chunks of `chunk` entries per row:
-// workgroup (row, chunk) writes its chunk's best min(k, count) as (order key, position).
-template <int NT, int J, bool LISTS>
+// kStripeLists: stage 1 of the two-stage selection (below) over `chunks` chunks of `chunk` entries per
+// row: workgroup (row, chunk) writes its chunk's best min(k, count) as (order key, position).
+// kStripeBlocks: select_candidate_blocks (candidate_kernel's result) at 8 scores per block: entries are
+// the blocks, an entry's key that of its maximum (+inf for the row's pinned last visible block), and
+// the output the keep bytes of all the row's scores.
+constexpr int kStripeRows = 0, kStripeLists = 1, kStripeBlocks = 2;
+
+// Four scores, four keep words: rows start anywhere (nb odd), so their pieces are only as aligned as
+// their elements, which global loads and stores allow.
+typedef float f32x4_row __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2_row __attribute__((ext_vector_type(2), aligned(1)));
+
+// The largest of block blk's scores in a row x of nb, 8 scores per block; NaNs are passed over. A block
+// of nothing but NaN gives NaN (nan_blocks) or -inf.
+__device__ __forceinline__ float block8_max(const float* x, int blk, int nb, bool nan_blocks) {
+  float m = -INFINITY;
+  if (blk * 8 + 8 <= nb) {
+    const f32x4_row u = *reinterpret_cast<const f32x4_row*>(x + blk * 8);
+    const f32x4_row v = *reinterpret_cast<const f32x4_row*>(x + blk * 8 + 4);
+    m = fmaxf(fmaxf(fmaxf(u[0], u[1]), fmaxf(u[2], u[3])), fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])));
+    return nan_blocks ? m : fmaxf(m, -INFINITY);
+  }
+  for (int t = blk * 8; t < nb; ++t) m = fmaxf(m, x[t]);
+  return m;
+}
+
+// Block blk's keep bytes.
+__device__ __forceinline__ void block8_keep(uint8_t* kr, int blk, int nb, bool keep) {
+  if (blk * 8 + 8 <= nb) {
+    const uint32_t w = keep ? 0x01010101u : 0u;
+    *reinterpret_cast<u32x2_row*>(kr + blk * 8) = u32x2_row{w, w};
+    return;
+  }
+  for (int t = blk * 8; t < nb; ++t) kr[t] = keep ? 1 : 0;
+}
+
+template <int NT, int J, int MODE>
 __global__ __launch_bounds__(NT, 8) void topk_stripe_kernel(
     const float* __restrict__ scores, int32_t* __restrict__ out, int n, int row_len, int k_max, int start_pos,
-    int ratio, int offset, int chunks, int chunk, uint32_t* __restrict__ ckey, int32_t* __restrict__ cpos) {
+    int ratio, int offset, int chunks, int chunk, uint32_t* __restrict__ ckey, int32_t* __restrict__ cpos,
+    uint8_t* __restrict__ keep, const int32_t* __restrict__ lens_v, int nan_blocks) {
+  constexpr bool LISTS = MODE == kStripeLists, BLOCKS = MODE == kStripeBlocks;
   constexpr int NBIN = 2048, NW = NT / 64, BPT = NBIN / NT;
   static_assert(BPT % 2 == 0, "a thread's bins are read 8 bytes at a time");
   __shared__ __align__(16) StripeShared<NT> sh;
   const uint32_t row = LISTS ? blockIdx.x / (unsigned)chunks : blockIdx.x;
   const int ch = LISTS ? (int)(blockIdx.x - row * (unsigned)chunks) : 0;
-  const int nb = LISTS ? min(chunk, row_len - ch * chunk) : row_len;   // entries of this selection
+  const int nb = LISTS ? min(chunk, row_len - ch * chunk)              // entries of this selection
+                       : (BLOCKS ? (row_len + 7) / 8 : row_len);
   const int k = LISTS ? min(k_max, nb) : k_max;
   const char* x = reinterpret_cast<const char*>(scores + (int64_t)row * row_len + ch * chunk);
   char* o = reinterpret_cast<char*>(out + (int64_t)row * k);
   const int64_t list = (int64_t)blockIdx.x * k_max;   // this chunk's list (LISTS)
   const int s = (int)(row % (unsigned)n);   // 32 bits: the 64-bit division is a long scalar routine
-  const int lens = (start_pos + s + 1) / ratio;
+  const int lens = BLOCKS && lens_v ? lens_v[s] : (start_pos + s + 1) / ratio;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if constexpr (LISTS) {
@@ -287,13 +324,18 @@ __global__ __launch_bounds__(NT, 8) void topk_stripe_kernel(
       return;
     }
   }
+  const int pinned = BLOCKS && lens > 0 ? (lens - 1) / 8 : -1;
   int p0 = wave * (64 * J) + lane;                 // this lane's first position
   // The positions p0 + 64 j are formed again where they are used: kept, they would take J registers.
   auto forget = [&]() { asm volatile("" : "+v"(p0)); };
   uint32_t key[J];
 #pragma unroll
   for (int j = 0; j < J; ++j) {
-    key[j] = __float_as_uint(*reinterpret_cast<const float*>(x + (uint32_t)min(p0 + 64 * j, nb - 1) * 4u));
+    if constexpr (BLOCKS)
+      key[j] = __float_as_uint(block8_max(reinterpret_cast<const float*>(x), min(p0 + 64 * j, nb - 1), row_len,
+                                           nan_blocks != 0));
+    else
+      key[j] = __float_as_uint(*reinterpret_cast<const float*>(x + (uint32_t)min(p0 + 64 * j, nb - 1) * 4u));
     if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);     // no more than 4 entries' temporaries at once
   }
   auto clear = [&](int b) {
@@ -307,6 +349,8 @@ __global__ __launch_bounds__(NT, 8) void topk_stripe_kernel(
 #pragma unroll
   for (int j = 0; j < J; ++j) {
     key[j] = p0 + 64 * j < nb ? order_key(__uint_as_float(key[j])) : 0u;
+    if constexpr (BLOCKS)                          // the pinned block
+      if (p0 + 64 * j == pinned) key[j] = kInfKey;
     if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
   }
   __syncthreads();
@@ -425,7 +469,10 @@ __global__ __launch_bounds__(NT, 8) void topk_stripe_kernel(
   auto emit = [&](uint64_t m, bool take, uint32_t base, int j) {
     const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, base));
     const int p = p0 + 64 * j;
-    if constexpr (LISTS) {
+    if constexpr (BLOCKS) {                        // a block of nothing but -inf or NaN is never kept
+      if (p < nb)
+        block8_keep(keep + (int64_t)row * row_len, p, row_len, take && key[j] > kNegInfKey && key[j] <= kInfKey);
+    } else if constexpr (LISTS) {
       if (take) {
         *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(ckey + list) + (rank << 2)) = key[j];
         *reinterpret_cast<int32_t*>(reinterpret_cast<char*>(cpos + list) + (rank << 2)) = ch * chunk + p;
@@ -504,6 +551,11 @@ __global__ __launch_bounds__(kSelThreads) void topk_kernel(const float* __restri
 }
 
 constexpr int kMaxCandBlocks = 8192;
+// Rows from which candidate blocks of 8 scores run on topk_stripe_kernel, us candidate_kernel -> stripe
+// (rows of 32,768 scores, 2,048 blocks kept): 64 rows 11.2 -> 10.3, 384 rows 21.8 ->
+// 15.9, 2,048 rows 99.0 -> 63.6; 1,400 x 22,804 417 us with byte stores and scalar reads of the rows
+// that are not 16-byte pieces, 52 us with element-aligned ones, 33.6 us on the stripe kernel.
+constexpr int64_t kCandStripeRows = 64;
 
 // select_candidate_blocks on the register core: thread t holds the maxima of blocks t*J ..
 // t*J+J-1 as order keys (the pinned block (lens-1)/bs as +inf); the best min(topk_blocks, nblk)
@@ -513,7 +565,7 @@ template <int J>
 __global__ __launch_bounds__(kSelThreads) void candidate_kernel(const float* __restrict__ scores,
                                                                 uint8_t* __restrict__ keep, int n, int nb,
                                                                 int topk_blocks, int bs, const int32_t* lens_v,
-                                                                int start_pos, int ratio, int vec8) {
+                                                                int start_pos, int ratio, int nan_blocks) {
   __shared__ RegSelShared sh;
   __shared__ uint8_t marked[kMaxCandBlocks];
   const int64_t row = blockIdx.x;
@@ -531,10 +583,8 @@ __global__ __launch_bounds__(kSelThreads) void candidate_kernel(const float* __r
     float m = -INFINITY;
     const int blk = j0 + j;
     if (j < nvalid) {
-      if (vec8 && blk * 8 + 8 <= nb) {                 // 8-score block, 16-byte aligned
-        const float4 u = *reinterpret_cast<const float4*>(x + blk * 8);
-        const float4 v = *reinterpret_cast<const float4*>(x + blk * 8 + 4);
-        m = fmaxf(fmaxf(fmaxf(u.x, u.y), fmaxf(u.z, u.w)), fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+      if (bs == 8) {
+        m = block8_max(x, blk, nb, nan_blocks != 0);
       } else {
         const int e = min(nb, (blk + 1) * bs);
         for (int t = blk * bs; t < e; ++t) m = fmaxf(m, x[t]);
@@ -559,9 +609,8 @@ __global__ __launch_bounds__(kSelThreads) void candidate_kernel(const float* __r
     if (j >= nvalid) continue;
     const int blk = j0 + j;
     const uint8_t v = (marked[blk] && bm[j] > -INFINITY) ? 1 : 0;
-    if (vec8 && blk * 8 + 8 <= nb) {
-      const uint32_t w = v ? 0x01010101u : 0u;
-      *reinterpret_cast<uint2*>(kr + blk * 8) = make_uint2(w, w);
+    if (bs == 8) {
+      block8_keep(kr, blk, nb, v != 0);
     } else {
       const int e = min(nb, (blk + 1) * bs);
       for (int t = blk * bs; t < e; ++t) kr[t] = v;
@@ -651,17 +700,22 @@ static TopkPlan topk_plan(int64_t rows, int nb, int k, bool allow_two_stage) {
 }
 
 // Launches topk_stripe_kernel for selections of at most `len` entries on a grid of one workgroup each.
-template <bool LISTS>
+template <int MODE>
 static void launch_stripe(int len, unsigned grid, const float* scores, int32_t* out, int n, int nb, int k,
                           int start_pos, int ratio, int offset, int chunks, int chunk, uint32_t* ckey, int32_t* cpos,
-                          hipStream_t stream) {
+                          uint8_t* keep, const int32_t* lens, int nan_blocks, hipStream_t stream) {
 #define DSV41_STRIPE_CASE(NT_, J_)                                                                                  \
   if (len <= NT_ * J_) {                                                                                            \
-    hipLaunchKernelGGL((topk_stripe_kernel<NT_, J_, LISTS>), dim3(grid), dim3(NT_), 0, stream, scores, out, n, nb, k, \
-                       start_pos, ratio, offset, chunks, chunk, ckey, cpos);                                        \
+    hipLaunchKernelGGL((topk_stripe_kernel<NT_, J_, MODE>), dim3(grid), dim3(NT_), 0, stream, scores, out, n, nb, k, \
+                       start_pos, ratio, offset, chunks, chunk, ckey, cpos, keep, lens, nan_blocks);                \
     return;                                                                                                         \
   }
-  if constexpr (!LISTS) {                          // chunks are longer than half of kStripeMax
+  if constexpr (MODE == kStripeBlocks) {           // at most kMaxCandBlocks
+    DSV41_STRIPE_CASE(256, 8)
+    DSV41_STRIPE_CASE(256, 16)
+    DSV41_STRIPE_CASE(512, 16)
+  }
+  if constexpr (MODE == kStripeRows) {             // chunks are longer than half of kStripeMax
     DSV41_STRIPE_CASE(256, 8)
     DSV41_STRIPE_CASE(256, 16)
     DSV41_STRIPE_CASE(256, 24)
@@ -670,9 +724,11 @@ static void launch_stripe(int len, unsigned grid, const float* scores, int32_t* 
     DSV41_STRIPE_CASE(512, 24)
     DSV41_STRIPE_CASE(512, 32)
   }
-  DSV41_STRIPE_CASE(512, 40)
-  DSV41_STRIPE_CASE(1024, 24)
-  DSV41_STRIPE_CASE(1024, 32)
+  if constexpr (MODE != kStripeBlocks) {
+    DSV41_STRIPE_CASE(512, 40)
+    DSV41_STRIPE_CASE(1024, 24)
+    DSV41_STRIPE_CASE(1024, 32)
+  }
 #undef DSV41_STRIPE_CASE
 }
 
@@ -705,8 +761,8 @@ static int topk_launch(const char* what, const float* scores, int32_t* out, int6
     int32_t* cpos = reinterpret_cast<int32_t*>(reinterpret_cast<uint8_t*>(workspace) + need / 2);
     const dim3 cgrid((unsigned)(rows * chunks));
     if (plan.stripe)
-      launch_stripe<true>(chunk, cgrid.x, scores, out, n, nb, k, start_pos, ratio, offset, chunks, chunk, ckey, cpos,
-                          stream);
+      launch_stripe<kStripeLists>(chunk, cgrid.x, scores, out, n, nb, k, start_pos, ratio, offset, chunks, chunk, ckey,
+                                  cpos, nullptr, nullptr, 0, stream);
     else if (chunk == kTopkChunk)
       hipLaunchKernelGGL(topk_chunk_kernel<kTopkChunk / kSelThreads>, cgrid, block, 0, stream, scores, ckey, cpos, nb, k,
                          chunks, vec);
@@ -718,7 +774,8 @@ static int topk_launch(const char* what, const float* scores, int32_t* out, int6
     return topk_merge_launch(what, ckey, cpos, out, rows, n, nb, k, chunks, chunk, start_pos, ratio, offset, stream);
   }
   if (plan.stripe) {
-    launch_stripe<false>(nb, grid.x, scores, out, n, nb, k, start_pos, ratio, offset, 1, nb, nullptr, nullptr, stream);
+    launch_stripe<kStripeRows>(nb, grid.x, scores, out, n, nb, k, start_pos, ratio, offset, 1, nb, nullptr, nullptr,
+                               nullptr, nullptr, 0, stream);
     return check_launch(what);
   }
   if (nb <= 4 * kSelThreads)
@@ -768,14 +825,18 @@ extern "C" int dsv41_candidate_blocks(const float* scores, uint8_t* keep, int64_
   DSV41_REQUIRE(rows < (1ll << 31), DSV41_E_ARG, "%s: too many rows", what);
   if (rows == 0 || nb == 0) return 0;
   const int nblk = (nb + block_size - 1) / block_size;
-  // 8-score blocks read as two float4 and written as 8 keep bytes: rows 16-byte aligned
-  const int vec8 = (block_size == 8 && nb % 4 == 0 && aligned16(scores) &&
-                    (reinterpret_cast<uintptr_t>(keep) & 7u) == 0 && nb % 8 == 0) ? 1 : 0;
+  // a whole block of NaNs counts as NaN where the rows are 16-byte pieces, else as -inf
+  const int nan_blocks = nb % 8 == 0 && aligned16(scores) && (reinterpret_cast<uintptr_t>(keep) & 7u) == 0 ? 1 : 0;
+  if (block_size == 8 && rows >= kCandStripeRows && topk_blocks > 0 && topk_blocks < nblk) {
+    launch_stripe<kStripeBlocks>(nblk, (unsigned)rows, scores, nullptr, n, nb, topk_blocks, start_pos, ratio, 0, 1, nb,
+                                 nullptr, nullptr, keep, lens, nan_blocks, stream);
+    return check_launch(what);
+  }
   if (nblk <= 4 * kSelThreads)
     hipLaunchKernelGGL(candidate_kernel<4>, dim3((unsigned)rows), dim3(kSelThreads), 0, stream, scores, keep, n, nb,
-                       topk_blocks, block_size, lens, start_pos, ratio, vec8);
+                       topk_blocks, block_size, lens, start_pos, ratio, nan_blocks);
   else
     hipLaunchKernelGGL(candidate_kernel<8>, dim3((unsigned)rows), dim3(kSelThreads), 0, stream, scores, keep, n, nb,
-                       topk_blocks, block_size, lens, start_pos, ratio, vec8);
+                       topk_blocks, block_size, lens, start_pos, ratio, nan_blocks);
   return check_launch(what);
 }

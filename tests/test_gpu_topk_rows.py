@@ -59,6 +59,23 @@ def test_rows_down_to_infinity_and_below(gpu, nb, k, inf):
     assert torch.equal(got, few)
 
 
+@pytest.mark.parametrize("rows,nb,kb", [
+    (512, 9, 1), (512, 4097, 300), (513, 16384, 2047), (520, 16385, 2048), (515, 22804, 2048),
+    (512, 32776, 4096), (512, 65536, 1),
+])
+@pytest.mark.parametrize("kind", ["normal", "ties", "masked", "odd"])
+def test_candidate_rows_equal_few_rows(gpu, rows, nb, kb, kind):
+    """Candidate blocks of many rows, 8 scores a block, against the same rows a few at a time."""
+    from dsv41 import _abi
+    x = _scores(rows, nb, kind)
+    x[7] = float("nan")                  # blocks of nothing but NaN
+    x[8, :, :64] = -float("nan")
+    lens = torch.tensor([nb - nb // 7], dtype=torch.int32, device="cuda")
+    got = _abi.candidate_blocks(x, kb, 8, lens)
+    few = torch.cat([_abi.candidate_blocks(x[i:i + 63].contiguous(), kb, 8, lens) for i in range(0, rows, 63)])
+    assert torch.equal(got, few)
+
+
 def test_rows_of_several_queries(gpu):
     """Visibility follows the query, row % n, also with rows of several sequences and k >= nb."""
     from dsv41 import _abi
