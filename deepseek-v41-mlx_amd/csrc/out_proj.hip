@@ -291,8 +291,17 @@ static void launch_wo_a(const WoaArgs& a, hipStream_t stream) {
     }
     return;
   }
-  if (a.r % kWideR == 0) launch_tiles<8, 4, 2, 4, 64, 2, TO>(a, stream);
-  else launch_tiles<4, 4, 2, 2, 64, 2, TO>(a, stream);
+  // Chunks: the largest tile that still gives most CUs one. 8 groups x (4096 -> 1024), us with
+  // 256 x 256 | 128 x 128, two per CU | 128 x 128, four stages | 64 x 128, three stages:
+  //    256 rows  105.8 | 56.6 | 42.9 | 33.8        1,024 rows  108.2 |  71.7 |  84.9 |  91.1
+  //    400 rows  105.1 | 57.7 | 43.8 | 48.9        1,300 rows  104.6 | 104.5 | 120.9 | 127.5
+  //    683 rows  107.1 | 63.9 | 81.4 | 73.6        4,096 rows  254.8 | 292.2 | 340.0 | 388.5
+  // Every tile sums the channels in the same order.
+  auto tiles = [&](int tr, int tm) { return (int64_t)a.groups * (a.r / tr) * ((a.rows + tm - 1) / tm); };
+  if (a.r % kWideR == 0 && tiles(256, 256) >= 192) launch_tiles<8, 4, 2, 4, 64, 2, TO>(a, stream);
+  else if (tiles(128, 128) > 256) launch_tiles<4, 4, 2, 2, 64, 2, TO>(a, stream);
+  else if (tiles(128, 128) > 128) launch_tiles<4, 4, 2, 2, 64, 4, TO>(a, stream);
+  else launch_tiles<2, 4, 2, 2, 64, 3, TO>(a, stream);
 }
 
 }  // namespace dsv41

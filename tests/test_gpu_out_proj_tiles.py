@@ -1,0 +1,27 @@
+"""The grouped output projection at chunk row counts, each tile shape against slices of decode row counts."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,groups,d,r", [
+    (129, 8, 512, 1024), (256, 8, 64, 1024),     # 64 x 128 tiles
+    (257, 8, 320, 1024), (511, 8, 512, 1024),    # 128 x 128, four stages; fewer steps than stages
+    (513, 8, 512, 1024), (1279, 8, 128, 1024),   # 128 x 128, two per CU
+    (1281, 8, 512, 1024), (1537, 8, 64, 1024),   # 256 x 256
+    (700, 3, 256, 384), (6000, 3, 128, 384),     # widths that are no multiple of 256
+])
+def test_chunk_rows_equal_decode_rows(gpu, rows, groups, d, r):
+    from dsv41 import _abi
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    o = torch.randn(rows, groups * d, generator=g, device="cuda").bfloat16()
+    w = torch.randn(groups * r, d, generator=g, device="cuda").bfloat16()
+    got = _abi.wo_a_grouped(o, w, groups, out_dtype=torch.float32)
+    few = torch.cat([_abi.wo_a_grouped(o[i:i + 128].contiguous(), w, groups, out_dtype=torch.float32)
+                     for i in range(0, rows, 128)])
+    assert torch.equal(got, few)
+    assert torch.equal(_abi.wo_a_grouped(o, w, groups), few.bfloat16())
