@@ -20,6 +20,8 @@ selection, without writing the scores.
 
 from __future__ import annotations
 
+import functools
+
 import numpy as np
 import torch
 
@@ -57,6 +59,7 @@ CHUNK_QUERIES = 8
 CHUNK_SCORES_FP8 = 1 << 19
 
 
+@functools.lru_cache(maxsize=256)
 def weight_scale(n_heads: int, head_dim: int, dtype) -> float:
     """head_dim**-0.5 * n_heads**-0.5 as the activation dtype holds it: a python scalar
     multiplying an MLX array takes the array's dtype (indexer.py:123)."""

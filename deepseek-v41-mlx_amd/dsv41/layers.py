@@ -46,13 +46,16 @@ def _decode_ok(lin: torch.nn.Linear, x: torch.Tensor) -> bool:
 
 def decode_linear(lin: torch.nn.Linear, x: torch.Tensor, wide_only: bool = False) -> torch.Tensor:
     """lin(x) on dsv41_linear_rows at decode row counts, else torch's linear. wide_only: only where
-    the 128-row tiles apply (the large projections wq_b and wo_b, 84 MB each at the release's
-    widths, where the 32-row tiles lose to the library: wo_b 32.8 against 29.0 us at 64 rows)."""
+    that is the faster one of the large projections (wq_b and wo_b, 84 MB each at the release's
+    widths): at 33-64 rows the 128-row tiles (on 32-row tiles wo_b takes 32.8 against 29.0 us at 64
+    rows), and up to 16 rows outputs wide enough to give every CU two 32-row tiles (wq_b
+    1280 -> 32768, weights streamed: 18.7-19.8 us against the library's 21.6-22.4 us, 20.7-21.6
+    against 19.9-20.1 us at 24 and 32 rows; wo_b 8192 -> 5120 23.4-26.8 against 19.7-21.5 us)."""
     if _decode_ok(lin, x):
         k, n = lin.weight.shape[1], lin.weight.shape[0]
         rows = x.numel() // k
         splits = _abi.linear_rows_splits(k, n, rows)
-        if not wide_only or _abi.linear_rows_wide(rows, k, n, splits):
+        if not wide_only or (rows <= 16 and n >= 512 * 32) or _abi.linear_rows_wide(rows, k, n, splits):
             return _abi.linear_rows(x.contiguous(), lin.weight, splits)
     return lin(x)
 

@@ -25,3 +25,18 @@ def test_chunk_rows_equal_decode_rows(gpu, rows, groups, d, r):
                      for i in range(0, rows, 128)])
     assert torch.equal(got, few)
     assert torch.equal(_abi.wo_a_grouped(o, w, groups), few.bfloat16())
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 33])
+def test_wide_projection_at_decode_rows(gpu, rows):
+    """A projection of at least 16,384 outputs, on either side of the row count where the library takes over."""
+    from dsv41.layers import decode_linear
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    lin = torch.nn.Linear(192, 16384, bias=False, dtype=torch.bfloat16, device="cuda")
+    lin.weight.data.normal_(generator=g)
+    x = torch.randn(rows, 192, generator=g, device="cuda").bfloat16()
+    got = decode_linear(lin, x, wide_only=True)
+    want = x.double() @ lin.weight.double().t()
+    # one rounding to bf16 (2^-8 of the value) of a float32 sum of 192 exact products
+    sums = 192 * 2 ** -23 * (x.double().abs() @ lin.weight.double().abs().t())
+    assert ((got.double() - want).abs() <= want.abs() * 2 ** -8 + sums).all()
