@@ -96,14 +96,14 @@ __device__ __forceinline__ void fake_quant_block(float* v) {
   if (FQ == FQ_FP8_UE8M0) {
     amax = fmaxf(amax, 1e-4f);
     const float s = pow2_ceil_log2(amax * (float)(1.0 / 448.0));
-    const float inv = __fdiv_rn(1.0f, s);   // s is a power of two: x * (1/s) rounds as x / s does
+    const float inv = pow2_inverse(s);      // s is a power of two: x * (1/s) rounds as x / s does
 #pragma unroll
     for (int i = 0; i < N; ++i)
       v[i] = io<T>::rnd(e4m3_round(fminf(fmaxf(v[i] * inv, -448.0f), 448.0f)) * s);
   } else if (FQ == FQ_FP4_UE8M0) {
     amax = fmaxf(amax, (float)(6.0 * 1.1754943508222875e-38));  // 6 * 2^-126
     const float s = pow2_ceil_log2(amax * (float)(1.0 / 6.0));
-    const float inv = __fdiv_rn(1.0f, s);   // s is a power of two: x * (1/s) rounds as x / s does
+    const float inv = pow2_inverse(s);      // s is a power of two: x * (1/s) rounds as x / s does
 #pragma unroll
     for (int i = 0; i < N; ++i)
       v[i] = io<T>::rnd(e2m1_round(fminf(fmaxf(v[i] * inv, -6.0f), 6.0f)) * s);
@@ -149,6 +149,9 @@ __device__ __forceinline__ RowPos row_pos(const RowArgs& a, int upr) {
   return p;
 }
 
+// Four consecutive floats at any element (rope tables start where the caller says).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 // EPT elements per thread: 32 / EPT lanes per 32-element chunk, lane `sub` of a chunk holding
 // elements sub * EPT .. +EPT of it.
 template <typename T, bool NORM, bool ROPE, int FQ, int BLK, int EPT, bool WIDE>
@@ -172,11 +175,25 @@ __global__ __launch_bounds__(256) void row_pipeline_kernel(RowArgs a) {
     const int64_t pos = (int64_t)a.pos_base + (int64_t)s * a.pos_step;
     const float* ct = a.cos_tab + pos * half;
     const float* st = a.sin_tab + pos * half;
+    if (first % EPT == 0) {                // uniform: the thread lies in the tail as a whole
+      const int p = (e0 - first) >> 1;
 #pragma unroll
-    for (int j = 0; j < EPT / 2; ++j) {
-      const int p = max(e0 + 2 * j - first, 0) >> 1;
-      cs[j] = ct[p];
-      sn[j] = st[p];
+      for (int j = 0; j < EPT / 2; j += 4) {
+        const f32x4_any c4 = *reinterpret_cast<const f32x4_any*>(ct + p + j);
+        const f32x4_any s4 = *reinterpret_cast<const f32x4_any*>(st + p + j);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          cs[j + i] = c4[i];
+          sn[j + i] = s4[i];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < EPT / 2; ++j) {
+        const int p = max(e0 + 2 * j - first, 0) >> 1;
+        cs[j] = ct[p];
+        sn[j] = st[p];
+      }
     }
   }
   float v[EPT];
@@ -302,9 +319,14 @@ static int launch_rows_ept(const RowArgs& a, hipStream_t stream, const char* wha
   return check_launch(what);
 }
 
-// 8 elements per thread, unless a fused norm would need more than 64 lanes for one row
+// 8 elements per thread, unless a fused norm would need more than 64 lanes for one row. A prompt's index
+// queries (a rope and no norm) take 16 once 8 would make 2^20 threads: the row's position costs three
+// integer divisions per thread (us at 8 | 16 | 32 elements: 8,192 x 64 heads 79.8 | 70.5 | 66.3, as
+// MXFP4 69.4 | 55.3 | 49.0; 2,048 x 32 heads 17.8 | 16.3 | 17.4).
 template <typename T, bool NORM, bool ROPE, int FQ, int BLK>
 static int launch_rows(const RowArgs& a, hipStream_t stream, const char* what) {
+  if constexpr (ROPE && !NORM && BLK == 32)
+    if (a.rows * a.cpr * 4 >= (int64_t)1 << 20) return launch_rows_ept<T, NORM, ROPE, FQ, BLK, 16>(a, stream, what);
   if (!NORM || a.cpr * 4 <= 64) return launch_rows_ept<T, NORM, ROPE, FQ, BLK, 8>(a, stream, what);
   return launch_rows_ept<T, NORM, ROPE, FQ, BLK, 32>(a, stream, what);
 }
