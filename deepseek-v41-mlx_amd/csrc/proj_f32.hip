@@ -217,6 +217,136 @@ __global__ __launch_bounds__(256) void proj_reduce_kernel(ProjArgs a) {
   store_proj(a, m, (int)(i - (int64_t)m * a.n), acc);
 }
 
+// The pooling of compress_pool_kernel (compress.hip: the same sums in the same order, the same state
+// update) straight from the projections, for 512 channels and ratio 2 or 4: a contraction cut into
+// ranges is summed here, range by range as proj_reduce_kernel does, so that kernel and its 4 bytes per
+// value out and back are gone, and a group's rows are read once, all at the same time, into registers
+// instead of three times one after another. Bound by the projections' bytes at chunk row counts and by
+// launches and load latency at decode ones. Against the two calls (us, k = 5120): 1 token 16.0 -> 13.1,
+// one of 32 sequences 19.6 -> 15.4, 300 tokens 34.8 -> 30.1, 1,000 66.0 -> 58.2, 8,191 228 -> 221.
+constexpr int kChunkDim = 512;
+
+struct ChunkArgs {
+  ProjArgs p;                            // splits > 1: the rows lie as parts, else in y0 and y1
+  float *kv_state, *score_state;         // [bsz, ratio, 512]
+  bf16_t* latents;                       // [bsz, g, 512]
+  const float* norm_w;
+  int n, m, g, rem;                      // tokens, carried rows, complete groups, rows left open
+  float eps;
+};
+
+// Channels tid + 256 u of NR projected rows: v[i][0] kv, v[i][1] score. Every load of up to four ranges
+// goes out before the first sum: a row at a time, each sum waited for its own loads (a token of 64
+// sequences 22.3 us against 14.6).
+constexpr int kChunkU = kChunkDim / 256;
+template <int NR>
+__device__ __forceinline__ void proj_values(const ProjArgs& a, const int (&row)[NR], int tid, float (&v)[NR][2][kChunkU]) {
+  const bool parts = a.splits > 1;
+  const int64_t total = (int64_t)a.rows * a.n;
+  const float* p[NR][2];
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int z = 0; z < 2; ++z) {
+      p[i][z] = parts ? a.part + (int64_t)row[i] * a.n + z * kChunkDim
+                      : (z ? a.y1 : a.y0) + (int64_t)row[i] * kChunkDim;
+#pragma unroll
+      for (int u = 0; u < kChunkU; ++u) v[i][z][u] = p[i][z][tid + 256 * u];
+    }
+  if (!parts) return;
+#pragma unroll 4
+  for (int s = 1; s < a.splits; ++s)
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+      for (int z = 0; z < 2; ++z)
+#pragma unroll
+        for (int u = 0; u < kChunkU; ++u) v[i][z][u] += (p[i][z] + s * total)[tid + 256 * u];
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int z = 0; z < 2; ++z)
+#pragma unroll
+      for (int u = 0; u < kChunkU; ++u)
+        if (__any(v[i][z][u] != v[i][z][u]) && v[i][z][u] != v[i][z][u])   // as store_proj
+          v[i][z][u] = plain_dot(a.x + (int64_t)row[i] * a.k, (z ? a.w1 : a.w0) + (int64_t)(tid + 256 * u) * a.k, a.k);
+}
+
+template <int R>
+__global__ __launch_bounds__(256) void compress_chunk_kernel(ChunkArgs a) {
+  constexpr int U = kChunkU;
+  __shared__ float red[4];
+  const int b = blockIdx.y, j = blockIdx.x, tid = threadIdx.x;
+  float* kst = a.kv_state + (int64_t)b * R * kChunkDim;
+  float* sst = a.score_state + (int64_t)b * R * kChunkDim;
+  if (a.g > 0) {
+    // rows j R .. of concat(state[:m], chunk); a carried one reads the chunk's first row and drops it
+    int row[R];
+    float v[R][2][U], carried[R][2][U];
+    const int held = max(a.m - j * R, 0);          // uniform: only group 0 meets carried rows
+#pragma unroll
+    for (int q = 0; q < R; ++q) row[q] = b * a.n + max(j * R + q - a.m, 0);
+    if (held > 0) {
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          carried[q][0][u] = kst[q * kChunkDim + tid + 256 * u];
+          carried[q][1][u] = sst[q * kChunkDim + tid + 256 * u];
+        }
+    }
+    proj_values<R>(a.p, row, tid, v);
+    if (held > 0) {
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[q][z][u] = q < held ? carried[q][z][u] : v[q][z][u];
+    }
+    float pooled[U], ss = 0.0f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int q = 0; q < R; ++q) mx = fmaxf(mx, v[q][1][u]);
+      float w[R], den = 0.0f;
+#pragma unroll
+      for (int q = 0; q < R; ++q) den += w[q] = expf(v[q][1][u] - mx);
+      float acc = 0.0f;
+#pragma unroll
+      for (int q = 0; q < R; ++q) acc += v[q][0][u] * (w[q] / den);
+      pooled[u] = io<bf16_t>::rnd(acc);  // rounded to the latents' type before the norm
+      ss += pooled[u] * pooled[u];
+    }
+    ss = group_sum(ss, 64);
+    if ((tid & 63) == 0) red[tid >> 6] = ss;
+    __syncthreads();
+    float tot = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) tot += red[w];
+    const float inv = 1.0f / sqrtf(tot / (float)kChunkDim + a.eps);
+    bf16_t* out = a.latents + ((int64_t)b * a.g + j) * kChunkDim;
+#pragma unroll
+    for (int u = 0; u < U; ++u) io<bf16_t>::st(out + tid + 256 * u, a.norm_w[tid + 256 * u] * (pooled[u] * inv));
+  }
+  // the open group's rows, by the workgroup that has read the carried ones (each thread its channels)
+  if (j == 0) {
+    for (int r = 0; r < a.rem; ++r) {
+      const int t = a.m + a.n - a.rem + r;
+      if (t < a.m) continue;             // a carried row, already in place
+      const int row[1] = {b * a.n + t - a.m};
+      float v[1][2][U];
+      proj_values<1>(a.p, row, tid, v);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        kst[r * kChunkDim + tid + 256 * u] = v[0][0][u];
+        sst[r * kChunkDim + tid + 256 * u] = v[0][1][u];
+      }
+    }
+  }
+}
+
 template <int WR, int WM, int GR, int GM>
 static void launch_proj(const ProjArgs& a, hipStream_t stream) {
   using C = ProjCfg<WR, WM, GR, GM>;
@@ -255,6 +385,26 @@ extern "C" size_t dsv41_linear_f32_pair_workspace_bytes(int32_t rows, int32_t k,
   return p.splits > 1 ? (size_t)p.splits * (size_t)rows * (size_t)n * sizeof(float) : 0;
 }
 
+// The checks of both entries below, then the projections: into y0 and y1, or into the workspace's parts.
+static int run_proj(const char* what, ProjArgs& a, const ProjPlan& p, size_t workspace_bytes, hipStream_t stream) {
+  DSV41_REQUIRE(a.k % 64 == 0 && a.n0 % 128 == 0 && (a.n - a.n0) % 128 == 0, DSV41_E_SHAPE,
+                "%s: k = %d must be a multiple of 64, n0 = %d and n1 = %d of 128", what, a.k, a.n0, a.n - a.n0);
+  DSV41_REQUIRE(aligned16(a.x) && aligned16(a.w0) && aligned16(a.w1) && aligned16(a.y0) && aligned16(a.y1), DSV41_E_ARG,
+                "%s: tensors must be 16-byte aligned", what);
+  DSV41_REQUIRE((int64_t)(a.n / p.tr) * p.splits * (((int64_t)a.rows + p.tm - 1) / p.tm) < (1ll << 31), DSV41_E_ARG,
+                "%s: too many tiles", what);
+  const size_t need = p.splits > 1 ? (size_t)p.splits * (size_t)a.rows * (size_t)a.n * sizeof(float) : 0;
+  DSV41_REQUIRE(workspace_bytes >= need && (need == 0 || (a.part && aligned16(a.part))), DSV41_E_WORKSPACE,
+                "%s: workspace of %zu bytes needed, %zu given", what, need, workspace_bytes);
+  a.splits = p.splits;
+  if (p.tr == 32) launch_proj<1, 1, 2, 2>(a, stream);
+  else if (p.tr == 64) launch_proj<1, 2, 4, 2>(a, stream);
+  else if (p.tm == 64) launch_proj<2, 2, 4, 2>(a, stream);
+  else if (p.tm == 128) launch_proj<2, 4, 4, 2>(a, stream);
+  else launch_proj<4, 4, 2, 4>(a, stream);
+  return check_launch(what);
+}
+
 extern "C" int dsv41_linear_f32_pair(const void* x, const float* w0, const float* w1, float* y0, float* y1,
                                      void* workspace, size_t workspace_bytes, int32_t rows, int32_t k, int32_t n0,
                                      int32_t n1, int32_t dtype, hipStream_t stream) {
@@ -262,27 +412,47 @@ extern "C" int dsv41_linear_f32_pair(const void* x, const float* w0, const float
   DSV41_REQUIRE(x && w0 && w1 && y0 && y1, DSV41_E_ARG, "%s: null tensor", what);
   DSV41_REQUIRE(dtype == DSV41_BF16, DSV41_E_DTYPE, "%s: bf16 activations only (dtype %d)", what, dtype);
   DSV41_REQUIRE(rows >= 0 && k > 0 && n0 > 0 && n1 > 0 && (int64_t)n0 + n1 < (1 << 24), DSV41_E_ARG, "%s: bad sizes", what);
-  DSV41_REQUIRE(k % 64 == 0 && n0 % 128 == 0 && n1 % 128 == 0, DSV41_E_SHAPE,
-                "%s: k = %d must be a multiple of 64, n0 = %d and n1 = %d of 128", what, k, n0, n1);
-  DSV41_REQUIRE(aligned16(x) && aligned16(w0) && aligned16(w1) && aligned16(y0) && aligned16(y1), DSV41_E_ARG,
-                "%s: tensors must be 16-byte aligned", what);
   if (rows == 0) return 0;
   const ProjPlan p = proj_plan(rows, k, n0 + n1);
-  DSV41_REQUIRE((int64_t)((n0 + n1) / p.tr) * p.splits * (((int64_t)rows + p.tm - 1) / p.tm) < (1ll << 31), DSV41_E_ARG,
-                "%s: too many tiles", what);
-  const size_t need = dsv41_linear_f32_pair_workspace_bytes(rows, k, n0, n1);
-  DSV41_REQUIRE(workspace_bytes >= need && (need == 0 || (workspace && aligned16(workspace))), DSV41_E_WORKSPACE,
-                "%s: workspace of %zu bytes needed, %zu given", what, need, workspace_bytes);
-  ProjArgs a{static_cast<const bf16_t*>(x), w0, w1, y0, y1, static_cast<float*>(workspace), rows, k, n0 + n1, n0,
-             p.splits};
-  if (p.tr == 32) launch_proj<1, 1, 2, 2>(a, stream);
-  else if (p.tr == 64) launch_proj<1, 2, 4, 2>(a, stream);
-  else if (p.tm == 64) launch_proj<2, 2, 4, 2>(a, stream);
-  else if (p.tm == 128) launch_proj<2, 4, 4, 2>(a, stream);
-  else launch_proj<4, 4, 2, 4>(a, stream);
-  int rc = check_launch(what);
+  ProjArgs a{static_cast<const bf16_t*>(x), w0, w1, y0, y1, static_cast<float*>(workspace), rows, k, n0 + n1, n0, 1};
+  const int rc = run_proj(what, a, p, workspace_bytes, stream);
   if (rc || p.splits <= 1) return rc;
   const int64_t quads = (int64_t)rows * a.n / 4;
   hipLaunchKernelGGL(proj_reduce_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, a);
+  return check_launch(what);
+}
+
+extern "C" size_t dsv41_compress_chunk_workspace_bytes(int32_t rows, int32_t k, int32_t dim) {
+  const size_t parts = dsv41_linear_f32_pair_workspace_bytes(rows, k, dim, dim);
+  return parts ? parts : (rows > 0 && dim > 0 ? 2 * (size_t)rows * (size_t)dim * sizeof(float) : 0);
+}
+
+extern "C" int dsv41_compress_chunk(const void* x, const float* w0, const float* w1, float* kv_state, float* score_state,
+                                    void* latents, const float* norm_w, void* workspace, size_t workspace_bytes,
+                                    int32_t bsz, int32_t n, int32_t k, int32_t dim, int32_t ratio, int32_t start_pos,
+                                    float eps, int32_t dtype, hipStream_t stream) {
+  const char* what = "dsv41_compress_chunk";
+  DSV41_REQUIRE(x && w0 && w1 && kv_state && score_state && norm_w, DSV41_E_ARG, "%s: null tensor", what);
+  DSV41_REQUIRE(dtype == DSV41_BF16, DSV41_E_DTYPE, "%s: bf16 activations only (dtype %d)", what, dtype);
+  DSV41_REQUIRE(bsz >= 0 && bsz < 65536 && n >= 0 && k > 0 && start_pos >= 0 && (int64_t)bsz * n < (1ll << 31), DSV41_E_ARG,
+                "%s: bad sizes", what);
+  DSV41_REQUIRE(dim == kChunkDim && (ratio == 2 || ratio == 4), DSV41_E_SHAPE,
+                "%s: dim %d and ratio %d (%d channels, ratio 2 or 4)", what, dim, ratio, kChunkDim);
+  const int rows = bsz * n;
+  if (rows == 0) return 0;
+  const int m = start_pos % ratio, total = m + n, g = total / ratio;
+  DSV41_REQUIRE(g == 0 || latents, DSV41_E_ARG, "%s: latents is null but %d groups complete", what, g);
+  const size_t need = dsv41_compress_chunk_workspace_bytes(rows, k, dim);
+  DSV41_REQUIRE(workspace && aligned16(workspace) && workspace_bytes >= need, DSV41_E_WORKSPACE,
+                "%s: workspace of %zu bytes needed, %zu given", what, need, workspace_bytes);
+  const ProjPlan p = proj_plan(rows, k, 2 * dim);
+  float* ws = static_cast<float*>(workspace);
+  ChunkArgs c{{static_cast<const bf16_t*>(x), w0, w1, ws, ws + (size_t)rows * dim, ws, rows, k, 2 * dim, dim, 1},
+              kv_state, score_state, static_cast<bf16_t*>(latents), norm_w, n, m, g, total % ratio, eps};
+  const int rc = run_proj(what, c.p, p, workspace_bytes, stream);
+  if (rc) return rc;
+  const dim3 grid((unsigned)(g > 0 ? g : 1), (unsigned)bsz);
+  if (ratio == 2) hipLaunchKernelGGL(compress_chunk_kernel<2>, grid, dim3(256), 0, stream, c);
+  else hipLaunchKernelGGL(compress_chunk_kernel<4>, grid, dim3(256), 0, stream, c);
   return check_launch(what);
 }

@@ -101,6 +101,9 @@ _SIGNATURES = {
     "dsv41_linear_rows_pair": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _sz, _i32, _i32, _i32, _i32, _i32, _i32, _c_p],
     "dsv41_linear_f32_pair_workspace_bytes": [_i32, _i32, _i32, _i32],
     "dsv41_linear_f32_pair": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _sz, _i32, _i32, _i32, _i32, _i32, _c_p],
+    "dsv41_compress_chunk_workspace_bytes": [_i32, _i32, _i32],
+    "dsv41_compress_chunk": [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _sz, _i32, _i32, _i32, _i32, _i32, _i32,
+                             _f32, _i32, _c_p],
     "dsv41_comp_write_fp8": [_c_p, _c_p, _i64, _c_p, _i64, _i32, _c_p, _c_p, _i32, _i32, _i32, _i32, _i32, _i32,
                              _i32, _c_p],
     "dsv41_index_key_publish_fp8": [_c_p, _c_p, _i64, _c_p, _i64, _i32, _c_p, _c_p, _c_p, _i32, _i32, _i32, _i32,
@@ -116,6 +119,7 @@ _RESTYPES = {
     "dsv41_sparse_mla_workspace_bytes": _sz,
     "dsv41_linear_rows_workspace_bytes": _sz,
     "dsv41_linear_f32_pair_workspace_bytes": _sz,
+    "dsv41_compress_chunk_workspace_bytes": _sz,
     "dsv41_topk_workspace_bytes": _sz,
     "dsv41_indexer_topk_workspace_bytes": _sz,
     "dsv41_version": ctypes.c_char_p,
@@ -436,6 +440,32 @@ def compress_pool(kv, score, kv_state, score_state, norm_w, ratio, start_pos, ep
         raise ValueError(f"{name}: dtype {dtype} not supported")
     _call(name, _ptr(kv), _ptr(score), _ptr(kv_state), _ptr(score_state), _ptr(lat), _ptr(norm_w),
           b, n, d, ratio, start_pos, float(eps), code, _stream(kv))
+    return lat
+
+
+def compress_chunk(x, w0, w1, kv_state, score_state, norm_w, ratio, start_pos, eps):
+    """compress_pool of linear_f32_pair(x, w0, w1) in one call (512 channels, ratio 2 or 4): latents
+    [b, g, 512] in bf16, or None when no group completes; the state is updated in place."""
+    name = "dsv41_compress_chunk"
+    _gpu(name, x, w0, w1, kv_state, score_state, norm_w)
+    _contig(name, x, w0, w1, kv_state, score_state, norm_w)
+    if x.dtype != torch.bfloat16 or x.dim() != 3:
+        raise ValueError(f"{name}: x must be bfloat16 [b, n, k]")
+    b, n, k = x.shape
+    for w in (w0, w1):
+        if w.dtype != torch.float32 or w.dim() != 2 or w.shape[1] != k or w.shape != w0.shape:
+            raise ValueError(f"{name}: the weights must be float32 [dim, {k}], got {w.dtype} {tuple(w.shape)}")
+    d = w0.shape[0]
+    for st in (kv_state, score_state):
+        if st.dtype != torch.float32 or st.dim() != 3 or st.shape[0] < b or st.shape[1:] != (ratio, d):
+            raise ValueError(f"{name}: state {st.dtype} {tuple(st.shape)} does not match float32 [>={b}, {ratio}, {d}]")
+    _vec(name, "norm weight", norm_w, d)
+    g = (start_pos % ratio + n) // ratio
+    lat = torch.empty(b, g, d, dtype=x.dtype, device=x.device) if g else None
+    need = lib().dsv41_compress_chunk_workspace_bytes(b * n, k, d)
+    ws = _workspace(need, x.device)
+    _call(name, _ptr(x), _ptr(w0), _ptr(w1), _ptr(kv_state), _ptr(score_state), _ptr(lat), _ptr(norm_w),
+          _ptr(ws), need, b, n, k, d, ratio, start_pos, float(eps), _DTYPES[x.dtype], _stream(x))
     return lat
 
 

@@ -1,7 +1,8 @@
 """Learned KV compression (deepseek_v41_mlx/compressor.py:36-88) on the GPU.
 
 * ratio > 1 (owner layers): ``kv = x @ wkv^T`` and ``score = x @ wgate^T`` in fp32 (bf16 activations:
-  one kernel for both, dsv41_linear_f32_pair; others: torch GEMMs), then one HIP kernel prepends the carried partial group,
+  one kernel for both, dsv41_linear_f32_pair, or both steps in one call, dsv41_compress_chunk; others:
+  torch GEMMs), then one HIP kernel prepends the carried partial group,
   pools every completed group with a per-channel softmax over the ratio axis, RMSNorms the
   pooled vector and stores the new remainder back into ``CompressorState``;
 * ratio == 1: a plain projection followed by the norm.
@@ -28,6 +29,9 @@ def _exact_weights_ok(x: torch.Tensor, w0: torch.Tensor, w1: torch.Tensor) -> bo
             and w0.data_ptr() % 16 == 0 and w1.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
 
 
+_CHUNK_DIM = 512     # the width dsv41_compress_chunk pools straight from the projections (ratio 2 or 4)
+
+
 class Compressor(torch.nn.Module):
     def __init__(self, args: ModelArgs, layer_id: int, dtype=torch.bfloat16, device="cuda"):
         super().__init__()
@@ -47,6 +51,9 @@ class Compressor(torch.nn.Module):
             return self.norm(self.wkv(x))
         w0, w1 = self.wkv.weight, self.wgate.weight
         if _exact_weights_ok(x, w0, w1):
+            if w0.shape[0] == w1.shape[0] == _CHUNK_DIM and self.ratio in (2, 4):
+                return _abi.compress_chunk(x.contiguous(), w0, w1, comp_state.kv_state, comp_state.score_state,
+                                           self.norm.weight, self.ratio, start_pos, self.norm.eps)
             kv, score = _abi.linear_f32_pair(x.contiguous(), w0, w1)
         else:
             xf = x.float()

@@ -155,6 +155,17 @@ int dsv41_linear_f32_pair(const void* x, const float* w0, const float* w1, float
                           void* workspace, size_t workspace_bytes, int32_t rows, int32_t k, int32_t n0,
                           int32_t n1, int32_t dtype, hipStream_t stream);
 
+/* dsv41_linear_f32_pair and dsv41_compress_pool in one call, deepseek_v41_mlx/compressor.py:58-79, for
+ * bf16 x [bsz, n, k], float32 weights w0, w1 [dim, k], dim 512 and ratio 2 or 4: the same latents and
+ * state, bit for bit, without the projected rows as tensors. rows = bsz * n; the workspace is
+ * dsv41_compress_chunk_workspace_bytes(...) bytes, 16-byte aligned. */
+size_t dsv41_compress_chunk_workspace_bytes(int32_t rows, int32_t k, int32_t dim);
+int dsv41_compress_chunk(const void* x, const float* w0, const float* w1, float* kv_state,
+                         float* score_state, void* latents, const float* norm_w, void* workspace,
+                         size_t workspace_bytes, int32_t bsz, int32_t n, int32_t k, int32_t dim,
+                         int32_t ratio, int32_t start_pos, float eps, int32_t dtype,
+                         hipStream_t stream);
+
 /* The compressed-cache write of Attention.__call__, deepseek_v41_mlx/attention.py:157-163:
  * comp_kv[b, g0 + j] <- fake_quant_fp4_e4m3(rope_tail(latents[b, j], position (g0+j)*ratio), 16)
  * for latents [bsz, g, dim]; comp_kv has `cache_bstride` elements per batch row. */

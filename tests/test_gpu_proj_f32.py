@@ -64,3 +64,29 @@ def test_compressor_shapes_outside_the_kernel(gpu):
     assert not _exact_weights_ok(x, w0, w1)
     x, w0, w1 = _data(4, 128, 128, 128, 2)
     assert _exact_weights_ok(x, w0, w1) and not _exact_weights_ok(x.float(), w0, w1)
+
+
+@pytest.mark.parametrize("b,n,start,ratio,k", [
+    (1, 1, 1, 2, 64),                    # one token closes a group; one contraction range
+    (32, 1, 4095, 4, 5120), (3, 1, 4094, 4, 5120),       # the second leaves its group open
+    (1, 300, 401, 2, 5120), (2, 77, 6, 4, 1024), (5, 3, 0, 4, 320),
+    (1, 1025, 7, 4, 640), (1, 4099, 2, 4, 128),          # one range at the last size: no parts
+])
+def test_chunk_equals_projections_and_pool(gpu, b, n, start, ratio, k):
+    from dsv41 import _abi
+    x, w0, w1 = _data(b * n, k, 512, 512, n + k)
+    x = x.view(b, n, k)
+    if n == 77:
+        x[1, 3, 5], x[0, 9, 2] = float("inf"), float("nan")
+        w1[7, 3] = float("-inf")
+    g = torch.Generator(device="cuda").manual_seed(n)
+    st = [torch.randn(b + 1, ratio, 512, generator=g, device="cuda") for _ in range(2)]
+    st2 = [t.clone() for t in st]
+    norm = torch.rand(512, generator=g, device="cuda") + 0.5
+    kv, score = _abi.linear_f32_pair(x, w0, w1)
+    want = _abi.compress_pool(kv, score, *st, norm, ratio, start, 1e-6, torch.bfloat16)
+    got = _abi.compress_chunk(x, w0, w1, *st2, norm, ratio, start, 1e-6)
+    assert (want is None) == (got is None)
+    for a, c in zip(([] if want is None else [want]) + st, ([] if got is None else [got]) + st2):
+        assert torch.equal(a.isnan(), c.isnan())
+        assert torch.equal(a.nan_to_num(7.0), c.nan_to_num(7.0))
