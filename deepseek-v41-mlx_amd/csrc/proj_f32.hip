@@ -12,8 +12,8 @@
 // Bound by the matrix cores at chunk row counts (3 x 2 rows k n multiply-adds on the bf16 rate, a
 // sixteenth of which is what float32 MFMAs reach) and by the weight stream (4 bytes each) at decode
 // row counts. Both projections, k = 5120, n = 512 + 512, against the library (x widened to float32,
-// then two float32 GEMMs): 8,191 rows 616 -> 236 us (1,090 TFLOP/s of bf16 products), 2,048 rows 173 ->
-// 81 us, 64 rows 28.6 -> 15.5 us, 1 row 26.5 -> 13.6 us.
+// then two float32 GEMMs), us: 8,191 rows 616 -> 216, 2,000 rows 173 -> 68, 64 rows 28.6 -> 15.5,
+// 1 row 26.5 -> 13.1 (1,190 TFLOP/s of bf16 products at 8,191 rows).
 //
 // A workgroup owns TR weight rows (of the two weights stacked) x TM activation rows and walks 64
 // channels per step, double-buffered. The activations arrive by LDS copies; the weights pass through
@@ -106,7 +106,8 @@ __global__ __launch_bounds__(64 * GR * GM, (ProjCfg<WR, WM, GR, GM>::LDS <= 80 *
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = (wave % GR) * 16 * WR, wm = (wave / GR) * 16 * WM;   // this wave's block
-  const int kr = a.k / a.splits;                      // channels of this range
+  const int steps = a.k / C::BK, first = sp * steps / a.splits;
+  const int nk = (sp + 1) * steps / a.splits - first; // 64-channel steps of this range
   // weights: wave w loads tile rows w TR/NWV + 4 j + g, lane l16 the channels 4 l16 .. + 3 of a step
   const float* wsrc[C::WL];
   int wdst[C::WL];
@@ -115,7 +116,7 @@ __global__ __launch_bounds__(64 * GR * GM, (ProjCfg<WR, WM, GR, GM>::LDS <= 80 *
     const int row = wave * (C::TR / C::NWV) + 4 * j + g;
     const int all = rt * C::TR + row;
     const float* base = all < a.n0 ? a.w0 + (int64_t)all * a.k : a.w1 + (int64_t)(all - a.n0) * a.k;
-    wsrc[j] = base + (int64_t)sp * kr + 4 * l16;
+    wsrc[j] = base + (int64_t)first * C::BK + 4 * l16;
     wdst[j] = row * C::RB + (((l16 >> 1) ^ proj_swz(row)) << 4) + 8 * (l16 & 1);
   }
   uint64_t xsrc[C::XL];
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(64 * GR * GM, (ProjCfg<WR, WM, GR, GM>::LDS <= 80 *
   for (int j = 0; j < C::XL; ++j) {
     const int row = wave * (C::TM / C::NWV) + 8 * j + (lane >> 3);
     const int64_t m = min(mt * C::TM + row, a.rows - 1);              // rows past the end: not stored
-    xsrc[j] = reinterpret_cast<uint64_t>(a.x + m * a.k + (int64_t)sp * kr + 8 * ((lane & 7) ^ proj_swz(row)));
+    xsrc[j] = reinterpret_cast<uint64_t>(a.x + m * a.k + (int64_t)first * C::BK + 8 * ((lane & 7) ^ proj_swz(row)));
   }
   const uint32_t lds0 = lds_offset(lds);
   auto issue_x = [&](int buf, int kt) {
@@ -155,7 +156,6 @@ __global__ __launch_bounds__(64 * GR * GM, (ProjCfg<WR, WM, GR, GM>::LDS <= 80 *
 #pragma unroll
     for (int j = 0; j < WM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int nk = kr / C::BK;
   issue_x(0, 0);
   load_w(0);
   store_w(0);
@@ -358,18 +358,39 @@ struct ProjPlan {
   int tr, tm, splits;
 };
 
-// Tiles as large as still give the chip a workgroup per CU (8 weight tiles at n = 1024), then as many
-// contraction ranges as fit one round of 256 workgroups: large tiles cut and read a weight for more
-// rows, short ranges fill the chip when rows are few.
+// Decode row counts: small tiles and as many contraction ranges as fit one round of 256 workgroups
+// (one per CU). Chunks: of three activation tiles and up to 40 ranges the pair with the least time as
+// measured per part (k = 5120, n = 1024): a round of workgroups takes 1.25, 1.66 or 2.56 us per
+// 64-channel step with 64, 128 or 256 activation rows, and 3 us to start and end; each range's partial
+// sums cost a write and a read at 5 TB/s. Within a few us of every size timed: 300 rows 29.4 -> 25.5 us,
+// 1,000 rows 58.5 -> 42.0, 2,500 rows 137.6 -> 83.4, 4,096 rows 140.9 -> 117.4, 5,000 rows 207 -> 157.7 (before: the
+// tile by row count alone, ranges of equal length only).
 static ProjPlan proj_plan(int rows, int k, int n) {
+  const int steps = k / 64;
+  if (rows <= 128) {
+    const int t = rows <= 32 ? 32 : 64;
+    ProjPlan p{t, t, 1};
+    const int64_t tiles = (int64_t)(n / p.tr) * ((rows + p.tm - 1) / p.tm);
+    for (int s = 2; s <= 40; ++s)
+      if (steps % s == 0 && tiles * s <= 256) p.splits = s;
+    return p;
+  }
+  static const int kRows[3] = {64, 128, 256};
+  static const double kStepUs[3] = {1.25, 1.66, 2.56};
   ProjPlan p{128, 256, 1};
-  if (rows <= 32) { p.tr = 32; p.tm = 32; }
-  else if (rows <= 128) { p.tr = 64; p.tm = 64; }
-  else if (rows <= 1024) p.tm = 64;
-  else if (rows <= 4096) p.tm = 128;
-  const int64_t tiles = (int64_t)(n / p.tr) * ((rows + p.tm - 1) / p.tm);
-  for (int s = 2; s <= 40; ++s)                        // ranges of whole 64-channel steps, one wave of the chip
-    if (k % (64 * s) == 0 && tiles * s <= 256) p.splits = s;
+  double best = 1e30;
+  for (int t = 0; t < 3; ++t) {
+    const int64_t tiles = (int64_t)(n / 128) * ((rows + kRows[t] - 1) / kRows[t]);
+    for (int s = 1; s <= 40 && s <= steps; ++s) {
+      const double us = (double)((tiles * s + 255) / 256) * ((steps + s - 1) / s * kStepUs[t] + 3.0) +
+                        (s > 1 ? (double)s * rows * n * 8.0 / 5e6 : 0.0);
+      if (us < best) {
+        best = us;
+        p.tm = kRows[t];
+        p.splits = s;
+      }
+    }
+  }
   return p;
 }
 

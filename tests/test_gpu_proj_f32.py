@@ -90,3 +90,15 @@ def test_chunk_equals_projections_and_pool(gpu, b, n, start, ratio, k):
     for a, c in zip(([] if want is None else [want]) + st, ([] if got is None else [got]) + st2):
         assert torch.equal(a.isnan(), c.isnan())
         assert torch.equal(a.nan_to_num(7.0), c.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("rows,k", [(129, 320), (700, 832), (1300, 448), (2500, 5120), (5000, 1088)])
+def test_ranges_of_unequal_length(gpu, rows, k):
+    """Row counts whose ranges do not divide the contraction's steps evenly."""
+    from dsv41 import _abi
+    x, w0, w1 = _data(rows, k, 512, 512, rows)
+    for y, w in zip(_abi.linear_f32_pair(x, w0, w1), (w0, w1)):
+        exact = x.double() @ w.double().t()
+        bound = (3 * k / 32 + 40) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())   # as above
+        assert bool(((y.double() - exact).abs() <= bound).all())
+        assert (y.double() - exact).norm() <= 1.05 * (F.linear(x.float(), w).double() - exact).norm()
