@@ -1155,11 +1155,20 @@ struct MlaPlan {
 // ~2 workgroups per CU). Splits of at most kPairList entries with head_dim <= 512 run the PAIR
 // instance (~77 KB of LDS, a two-slot ring), the rest one ~160 KB workgroup per CU. A workgroup
 // stages at most kMaxList list entries.
+//
+// The two-role kernel (512 channels, whole 64-head groups) takes over past 128 of its workgroups: up to
+// there four splits per 32-head unit fill the chip evenly, past it two uneven rounds of long splits
+// would run. us, split lists -> two-role kernel, 64 heads:
+//   640 rows, bf16:    96 queries 36.8 -> 38.2, 130 59.5 -> 39.1, 200 77.9 -> 40.5, 240 76.1 -> 36.2
+//   640 rows, packed:  96 queries 52.1 -> 79.1, 130 123.0 -> 79.4, 200 162.5 -> 80.3
+//   2,176 rows, bf16:  128 queries 101.6 -> 79.3, 200 191.2 -> 80.0
+//   window only, bf16: 128 tokens 20.2 -> 23.8, 130 queries 25.6 -> 23.7, 200 29.7 -> 24.3
 static MlaPlan plan_bf16(int64_t units, int heads, int list_max, int dim) {
   MlaPlan p{};
   const int lm = list_max > 0 ? list_max : 1;
   const int hg32 = (heads + 31) / 32;
-  if (units * hg32 >= 512 && lm <= kMaxList) {
+  const bool roles = dim == 512 && heads % 64 == 0 && units * (heads / 64) > 128;
+  if ((units * hg32 >= 512 || roles) && lm <= kMaxList) {
     p.wide = heads > 32;
     p.hgroups = p.wide ? (heads + 63) / 64 : hg32;
     p.splits = 1;
