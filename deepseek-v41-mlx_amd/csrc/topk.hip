@@ -324,7 +324,8 @@ __global__ __launch_bounds__(NT, 8) void topk_stripe_kernel(
       return;
     }
   }
-  const int pinned = BLOCKS && lens > 0 ? (lens - 1) / 8 : -1;
+  const int last = BLOCKS && lens > 0 ? (lens - 1) / 8 : -1;
+  const int pinned = last < nb ? last : -1;        // past the row's blocks: none, and no place taken
   int p0 = wave * (64 * J) + lane;                 // this lane's first position
   // The positions p0 + 64 j are formed again where they are used: kept, they would take J registers.
   auto forget = [&]() { asm volatile("" : "+v"(p0)); };

@@ -76,6 +76,19 @@ def test_candidate_rows_equal_few_rows(gpu, rows, nb, kb, kind):
     assert torch.equal(got, few)
 
 
+@pytest.mark.parametrize("nb,kb,past", [(1999, 100, 1), (1999, 100, 40), (4104, 64, 8), (16384, 2047, 300)])
+def test_candidate_rows_visible_past_their_end(gpu, nb, kb, past):
+    """A visibility beyond the row pins no block: all kb places go to the row's own blocks."""
+    from dsv41 import _abi
+    x = _scores(520, nb, "normal")
+    lens = torch.tensor([nb + past], dtype=torch.int32, device="cuda")
+    got = _abi.candidate_blocks(x, kb, 8, lens)
+    few = torch.cat([_abi.candidate_blocks(x[i:i + 63].contiguous(), kb, 8, lens) for i in range(0, 520, 63)])
+    assert torch.equal(got, few)
+    pad = torch.nn.functional.pad(got, (0, -nb % 8)).unflatten(-1, (-1, 8))
+    assert bool((pad.any(-1).sum(-1) == kb).all())
+
+
 def test_rows_of_several_queries(gpu):
     """Visibility follows the query, row % n, also with rows of several sequences and k >= nb."""
     from dsv41 import _abi
