@@ -672,15 +672,18 @@ constexpr int kStripeMax = 32 * kSelThreads;   // entries of the largest stripe 
 // on scores already in cache (17.5-19.3 against 19.4-20.2 us), but inside a decode step, reading
 // the scores the scoring kernel has just written, the two stages spread that read over 8
 // workgroups per row and win: the 40-layer fp8 step took 1.163-1.166 ms against 1.190-1.195 ms.
+static int64_t stripe_from(int nb) { return nb <= 16 * kSelThreads ? 512 : (nb <= kStripeMax ? 64 : 128); }
+
 static TopkPlan topk_plan(int64_t rows, int nb, int k, bool allow_two_stage) {
   TopkPlan p{false, 0, 0};
   if (k >= nb) return p;                           // everything is selected
+  const bool many = rows >= stripe_from(nb);
   if (nb <= kStripeMax) {
-    p.stripe = rows >= 512 || (nb > 16 * kSelThreads && rows >= 64);
+    p.stripe = many;
     if (p.stripe) return p;
   }
   if (!allow_two_stage || nb <= 16 * kSelThreads) return p;
-  if (nb > kStripeMax && rows >= 128) {
+  if (nb > kStripeMax && many) {
     const int c = (nb + kStripeMax - 1) / kStripeMax;
     const int ch = ((nb + c - 1) / c + 63) / 64 * 64;
     if (k <= ch && (int64_t)c * k <= 32 * kSelThreads && (int64_t)(c - 1) * ch < nb && rows * c < (1ll << 31)) {
@@ -750,7 +753,12 @@ static int topk_launch(const char* what, const float* scores, int32_t* out, int6
   if (rows == 0 || k == 0) return 0;
   const dim3 grid((unsigned)rows), block(kSelThreads);
   const int vec = (nb % 4 == 0 && aligned16(scores)) ? 1 : 0;
-  const TopkPlan plan = topk_plan(rows, nb, k, allow_two_stage);
+  TopkPlan plan = topk_plan(rows, nb, k, allow_two_stage);
+  // Many rows in two stages where few take one (k over half a chunk): a caller without the workspace still
+  // gets the one stage.
+  if (plan.chunks && !topk_plan(1, nb, k, true).chunks &&
+      !(workspace && aligned16(workspace) && workspace_bytes >= topk_ws_bytes(rows, plan.chunks, k)))
+    plan = TopkPlan{false, 0, 0};
   if (plan.chunks) {
     const int chunks = plan.chunks, chunk = plan.chunk;
     const size_t need = topk_ws_bytes(rows, chunks, k);
@@ -803,8 +811,15 @@ extern "C" int dsv41_topk_select(const float* scores, int32_t* out, int64_t rows
 extern "C" size_t dsv41_topk_workspace_bytes(int64_t rows, int32_t nb, int32_t topk) {
   if (rows <= 0 || nb <= 0 || topk <= 0) return 0;
   const int k = topk < nb ? topk : nb;
-  const TopkPlan p = topk_plan(rows, nb, k, true);
-  return p.chunks ? topk_ws_bytes(rows, p.chunks, k) : 0;
+  // At least what any smaller number of rows takes (few rows need more than many: from stripe_from on the
+  // chunks are fewer, or none), so that a workspace sized for the largest batch serves every batch.
+  auto bytes = [&](int64_t r) {
+    const TopkPlan p = topk_plan(r, nb, k, true);
+    return p.chunks ? topk_ws_bytes(r, p.chunks, k) : (size_t)0;
+  };
+  const int64_t few = stripe_from(nb) - 1;
+  const size_t own = bytes(rows), less = rows > few ? bytes(few) : 0;
+  return own > less ? own : less;
 }
 
 extern "C" int dsv41_topk_select_ws(const float* scores, int32_t* out, int64_t rows, int32_t n, int32_t nb,

@@ -358,7 +358,8 @@ int dsv41_topk_select(const float* scores, int32_t* out, int64_t rows, int32_t n
  * k <= 2048 when there are few rows, over 32768 when there are many) are then selected in two stages
  * (each chunk's best k, then the best k of those lists), spreading a row over several workgroups. The
  * workspace is dsv41_topk_workspace_bytes(rows, nb, topk) bytes, 16-byte aligned (0: one stage,
- * workspace may be null). */
+ * workspace may be null). The size never falls as rows grow: one workspace sized for the most rows
+ * serves every smaller call over the same nb and topk. */
 size_t dsv41_topk_workspace_bytes(int64_t rows, int32_t nb, int32_t topk);
 int dsv41_topk_select_ws(const float* scores, int32_t* out, int64_t rows, int32_t n, int32_t nb,
                          int32_t topk, int32_t start_pos, int32_t ratio, int32_t offset,

@@ -100,15 +100,40 @@ def test_rows_of_several_queries(gpu):
         assert torch.equal(got, few)
 
 
-def test_workspace_matches_the_route(gpu):
-    """Rows that one workgroup selects need no workspace; longer ones state theirs and refuse less."""
+def _select_ws(x, k, ws):
     from dsv41 import _abi
-    assert _abi.topk_workspace_bytes(2048, 32768, 512) == 0
-    need = _abi.topk_workspace_bytes(128, 65536, 512)
-    assert need == 2 * 128 * 2 * 512 * 4
+    rows, _, nb = x.shape
+    out = torch.empty(rows, 1, k, dtype=torch.int32, device="cuda")
+    _abi._call("dsv41_topk_select_ws", _abi._ptr(x), _abi._ptr(out), rows, 1, nb, k, 2 * nb, 1, 0, _abi._ptr(ws),
+               ws.numel() if ws is not None else 0, _abi._stream(x))
+    return out
+
+
+def test_workspace_matches_the_route(gpu):
+    """Two-stage rows state their workspace and refuse less than they use."""
+    from dsv41 import _abi
+    used = 2 * 128 * 2 * 512 * 4         # two chunks' lists of 512 keys and positions
+    assert _abi.topk_workspace_bytes(128, 65536, 512) >= used
     x = torch.randn(128, 1, 65536, device="cuda")
-    out = torch.empty(128, 1, 512, dtype=torch.int32, device="cuda")
-    small = torch.empty(need - 256, dtype=torch.uint8, device="cuda")
+    small = torch.empty(used - 256, dtype=torch.uint8, device="cuda")
     with pytest.raises(ValueError):
-        _abi._call("dsv41_topk_select_ws", _abi._ptr(x), _abi._ptr(out), 128, 1, 65536, 512, 70000, 1, 0,
-                   _abi._ptr(small), small.numel(), _abi._stream(x))
+        _select_ws(x, 512, small)
+
+
+@pytest.mark.parametrize("nb,k,most,fewer", [(32768, 512, 64, (63, 64, 31)), (32768, 512, 2048, (63, 600)),
+                                             (65536, 512, 128, (127, 128, 5)), (20001, 1024, 300, (63, 64, 300))])
+def test_workspace_of_the_most_rows_serves_fewer(gpu, nb, k, most, fewer):
+    from dsv41 import _abi
+    ws = torch.empty(_abi.topk_workspace_bytes(most, nb, k), dtype=torch.uint8, device="cuda")
+    x = _scores(max(fewer), nb, "normal")
+    for rows in fewer:
+        part = x[:rows].contiguous()
+        assert torch.equal(_select_ws(part, k, ws), _abi.topk_select(part, k, 2 * nb, 1, 0))
+
+
+def test_many_rows_without_a_workspace(gpu):
+    """k over half a chunk: few rows take one stage and no workspace, many take two only if they get one."""
+    from dsv41 import _abi
+    assert _abi.topk_workspace_bytes(127, 65536, 3000) == 0 < _abi.topk_workspace_bytes(128, 65536, 3000)
+    x = _scores(128, 65536, "ties")
+    assert torch.equal(_select_ws(x, 3000, None), _abi.topk_select(x, 3000, 131072, 1, 0))
