@@ -1163,11 +1163,11 @@ struct MlaPlan {
 //   640 rows, packed:  96 queries 52.1 -> 79.1, 130 123.0 -> 79.4, 200 162.5 -> 80.3
 //   2,176 rows, bf16:  128 queries 101.6 -> 79.3, 200 191.2 -> 80.0
 //   window only, bf16: 128 tokens 20.2 -> 23.8, 130 queries 25.6 -> 23.7, 200 29.7 -> 24.3
-static MlaPlan plan_bf16(int64_t units, int heads, int list_max, int dim) {
+static MlaPlan plan_bf16(int64_t units, int heads, int list_max, int dim, bool two_role = true) {
   MlaPlan p{};
   const int lm = list_max > 0 ? list_max : 1;
   const int hg32 = (heads + 31) / 32;
-  const bool roles = dim == 512 && heads % 64 == 0 && units * (heads / 64) > 128;
+  const bool roles = two_role && dim == 512 && heads % 64 == 0 && units * (heads / 64) > 128;
   if ((units * hg32 >= 512 || roles) && lm <= kMaxList) {
     p.wide = heads > 32;
     p.hgroups = p.wide ? (heads + 63) / 64 : hg32;
@@ -1292,7 +1292,11 @@ extern "C" size_t dsv41_sparse_mla_workspace_bytes(int32_t bsz, int32_t m, int32
                                                    int32_t rows_per_query, int32_t dtype) {
   if (dtype != DSV41_BF16 || bsz <= 0 || m <= 0 || heads <= 0 || dim <= 0) return 0;
   const int64_t units = (int64_t)bsz * m;
-  return workspace_for(plan_bf16(units, heads, rows_per_query, dim), units, heads, dim);
+  // What split lists take, also where the two-role kernel needs none: a buffer sized for 129-255 queries
+  // serves fewer, whose lists are split.
+  const size_t own = workspace_for(plan_bf16(units, heads, rows_per_query, dim), units, heads, dim);
+  const size_t split = workspace_for(plan_bf16(units, heads, rows_per_query, dim, false), units, heads, dim);
+  return own > split ? own : split;
 }
 
 extern "C" int dsv41_sparse_attn(const void* q, const void* kv, const float* sink, const int32_t* idx, void* o,

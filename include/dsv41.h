@@ -378,8 +378,10 @@ int dsv41_candidate_blocks(const float* scores, uint8_t* keep, int64_t rows, int
 /* ---------------------------------------------------------------- sparse MLA --
  */
 
-/* Scratch bytes the sparse-MLA entry points need for split partial results at this shape
- * (0 when no split is used). `rows_per_query` = window rows + index rows. */
+/* Scratch bytes for the split partial results of the sparse-MLA entry points at this shape (0 when no
+ * split is used). `rows_per_query` = window rows + index rows. At 129-255 (query, 64 heads) of 512
+ * channels the kernel itself needs none; the size stated there is that of split lists, so that one
+ * buffer also serves smaller batches. */
 size_t dsv41_sparse_mla_workspace_bytes(int32_t bsz, int32_t m, int32_t heads, int32_t dim,
                                         int32_t rows_per_query, int32_t dtype);
 
@@ -436,7 +438,7 @@ int dsv41_sparse_mla_decode(const void* q, void* win_kv, const void* chunk_kv,
  * No counterpart in the reference: its sparse_attn allocates its output and scratch per call.
  * Same arguments, result and ring write as dsv41_sparse_mla_decode. The split partials live in a
  * static 32 MiB device array inside the library, one per GPU, held until the process ends; a
- * shape whose split scratch (dsv41_sparse_mla_workspace_bytes) exceeds 32 MiB returns
+ * shape whose splits need more than 32 MiB (see dsv41_sparse_mla_workspace_bytes) returns
  * DSV41_E_WORKSPACE before any launch. Nothing is allocated or freed. Every call on one GPU shares
  * that GPU's array: calls that overlap on one GPU (different streams, no ordering between them)
  * race; calls ordered on one stream are safe (each call writes every partial it reads). */
