@@ -58,25 +58,20 @@ __device__ __forceinline__ Planes cut_weights(const float4 w) {
   return o;
 }
 
-// Infinities: an infinite weight leaves NaN behind its first plane, and an infinite activation
-// meets planes that are 0, so a result that should be infinite comes out NaN. A NaN result is
-// therefore formed again in plain float32 (never taken with finite inputs).
-__device__ __noinline__ float plain_dot(const bf16_t* x, const float* w, int k) {
-  float s = 0.0f;
-  for (int i = 0; i < k; ++i) s += bf2f(x[i]) * w[i];
-  return s;
+// Infinities: an infinite weight leaves NaN behind its first plane, and an infinite activation meets
+// planes that are 0, so a sum that should be infinite comes out NaN. NaN sums are therefore formed again
+// from what decides them alone: a weight counts as NaN, as an infinity, as 0 or as 2^-40 with its sign (so
+// that no finite sum overflows). Infinite there, the result is that infinity; else it stays NaN. Per wave
+// and 16 weight rows, from memory and on the matrix cores, so that rows full of NaN stay within a few times
+// the finite ones' time (one output at a time by one lane, each a serial loop over k, took thousands of
+// times as long).
+__device__ __forceinline__ uint32_t weight_class(uint32_t w) {   // bf16 bits
+  const uint32_t m = w & 0x7FFFFFFFu, s = (w >> 16) & 0x8000u;
+  return m > 0x7F800000u ? 0x7FC0u : (m == 0x7F800000u ? s | 0x7F80u : (m ? s | 0x2B80u : 0u));
 }
 __device__ __forceinline__ void store_proj(const ProjArgs& a, int m, int j, f32x4 v) {   // columns j .. j + 3 of row m
-  const bool second = j >= a.n0;
-  const int jj = second ? j - a.n0 : j;
-  if (__any(v[0] != v[0] || v[1] != v[1] || v[2] != v[2] || v[3] != v[3])) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (v[i] != v[i])
-        v[i] = plain_dot(a.x + (int64_t)m * a.k, (second ? a.w1 : a.w0) + (int64_t)(jj + i) * a.k, a.k);
-  }
-  float* y = second ? a.y1 + (int64_t)m * (a.n - a.n0) : a.y0 + (int64_t)m * a.n0;
-  *reinterpret_cast<f32x4*>(y + jj) = v;
+  float* y = j >= a.n0 ? a.y1 + (int64_t)m * (a.n - a.n0) + (j - a.n0) : a.y0 + (int64_t)m * a.n0 + j;
+  *reinterpret_cast<f32x4*>(y) = v;
 }
 
 // A GR x GM grid of waves, each 16 WR weight rows x 16 WM activation rows.
@@ -190,6 +185,44 @@ __global__ __launch_bounds__(64 * GR * GM, (ProjCfg<WR, WM, GR, GM>::LDS <= 80 *
   }
 
 #pragma unroll
+  for (int i = 0; i < WR; ++i) {
+    bool nan = false;
+#pragma unroll
+    for (int j = 0; j < WM; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) nan = nan || acc[i][j][e] != acc[i][j][e];
+    if (!__any(nan)) continue;                        // always, unless an input is infinite or NaN or a sum overflows
+    const int all = rt * C::TR + wr + 16 * i + l16;
+    const float* wrow = (all < a.n0 ? a.w0 + (int64_t)all * a.k : a.w1 + (int64_t)(all - a.n0) * a.k) +
+                        (int64_t)first * C::BK + 8 * g;
+    f32x4 dec[WM];
+#pragma unroll
+    for (int j = 0; j < WM; ++j) dec[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < nk * C::BK; c += 32) {
+      union {
+        uint32_t u[4];
+        bf16x8 v;
+      } af;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const uint4 w = *reinterpret_cast<const uint4*>(wrow + c + 4 * e);
+        af.u[2 * e] = weight_class(w.x) | weight_class(w.y) << 16;
+        af.u[2 * e + 1] = weight_class(w.z) | weight_class(w.w) << 16;
+      }
+#pragma unroll
+      for (int j = 0; j < WM; ++j) {
+        const int64_t m = min(mt * C::TM + wm + 16 * j + l16, a.rows - 1);
+        dec[j] = mfma16x16x32(af.v, ld_bf16x8(a.x + m * a.k + (int64_t)first * C::BK + c + 8 * g), dec[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < WM; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (acc[i][j][e] != acc[i][j][e] && fabsf(dec[j][e]) == INFINITY) acc[i][j][e] = dec[j][e];
+  }
+
+#pragma unroll
   for (int j = 0; j < WM; ++j) {
     const int m = mt * C::TM + wm + 16 * j + l16;
     if (m >= a.rows) continue;
@@ -262,14 +295,6 @@ __device__ __forceinline__ void proj_values(const ProjArgs& a, const int (&row)[
       for (int z = 0; z < 2; ++z)
 #pragma unroll
         for (int u = 0; u < kChunkU; ++u) v[i][z][u] += (p[i][z] + s * total)[tid + 256 * u];
-#pragma unroll
-  for (int i = 0; i < NR; ++i)
-#pragma unroll
-    for (int z = 0; z < 2; ++z)
-#pragma unroll
-      for (int u = 0; u < kChunkU; ++u)
-        if (__any(v[i][z][u] != v[i][z][u]) && v[i][z][u] != v[i][z][u])   // as store_proj
-          v[i][z][u] = plain_dot(a.x + (int64_t)row[i] * a.k, (z ? a.w1 : a.w0) + (int64_t)(tid + 256 * u) * a.k, a.k);
 }
 
 template <int R>

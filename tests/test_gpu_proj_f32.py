@@ -57,6 +57,50 @@ def test_projections_with_infinities(gpu):
         assert torch.equal(y[y.isinf()], lib[lib.isinf()])
 
 
+@pytest.mark.parametrize("rows,k", [(5, 5120), (70, 320), (300, 192), (1025, 448), (4097, 128)])
+def test_infinities_in_every_tile(gpu, rows, k):
+    """Infinite and NaN activations and weights against float64, per tile size and with ranges; every output
+    they do not reach keeps its bits."""
+    from dsv41 import _abi
+    x, w0, w1 = _data(rows, k, 128, 128, rows)
+    clean = _abi.linear_f32_pair(x, w0, w1)
+    x[0, 3], x[1, 70 % k], x[2, 9] = float("inf"), float("-inf"), float("nan")
+    x[rows - 1, 5], x[rows - 1, k - 1] = float("inf"), float("-inf")
+    w0[3, 11], w0[127, k - 2] = float("-inf"), float("inf")
+    w1[64, 20] = float("nan")
+    w1[5, 3], w1[6, 3], w1[7, 3] = 0.0, 1e-41, -1e-41       # times the infinite activation: NaN, inf, -inf
+    hit = x.float().isfinite().all(1, keepdim=True)
+    for y, w, c in zip(_abi.linear_f32_pair(x, w0, w1), (w0, w1), clean):
+        want = x.double() @ w.double().t()
+        assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.isposinf(), want.isposinf())
+        assert torch.equal(y.isneginf(), want.isneginf())
+        keep = hit & w.isfinite().all(1) & (torch.arange(128, device="cuda") > 7)
+        assert torch.equal(y[keep], c[keep])
+
+
+@pytest.mark.parametrize("rows", [64, 2000])
+def test_nan_rows_take_a_few_times_as_long_at_most(gpu, rows):
+    """A poisoned batch must not hold up the launch: one re-evaluation on the matrix cores (measured 2 to 5
+    times the finite time; the bound leaves room for a busy card)."""
+    from dsv41 import _abi
+
+    def best_us(x):
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        us = []
+        for _ in range(5):
+            e[0].record()
+            y = _abi.linear_f32_pair(x, w0, w1)
+            e[1].record()
+            torch.cuda.synchronize()
+            us.append(e[0].elapsed_time(e[1]) * 1e3)
+        return min(us), y[0]
+
+    x, w0, w1 = _data(rows, 5120, 512, 512, 1)
+    finite, _ = best_us(x)
+    poisoned, y = best_us(torch.full_like(x, float("nan")))
+    assert bool(y.isnan().all()) and poisoned < 20 * finite + 50
+
+
 def test_compressor_shapes_outside_the_kernel(gpu):
     """Widths that are not whole tiles and float32 activations keep torch's linear."""
     from dsv41.compressor import _exact_weights_ok
