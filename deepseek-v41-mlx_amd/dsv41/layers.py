@@ -44,18 +44,31 @@ def _decode_ok(lin: torch.nn.Linear, x: torch.Tensor) -> bool:
             and w.shape[1] % 64 == 0 and w.shape[0] % 32 == 0)
 
 
+def _only_the_product(lin: torch.nn.Linear, x: torch.Tensor) -> bool:
+    """Whether calling lin does nothing beyond the product (no hooks, no forward of its own, no gradient) on
+    tensors aligned for dsv41_linear_rows, so that the kernel may stand in for the module."""
+    mod = torch.nn.modules.module
+    return (type(lin).forward is torch.nn.Linear.forward and "forward" not in lin.__dict__
+            and not (lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks or lin._backward_pre_hooks
+                     or mod._global_forward_hooks or mod._global_forward_pre_hooks)
+            and not (torch.is_grad_enabled() and (x.requires_grad or lin.weight.requires_grad))
+            and lin.weight.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
+
+
 def decode_linear(lin: torch.nn.Linear, x: torch.Tensor, wide_only: bool = False) -> torch.Tensor:
     """lin(x) on dsv41_linear_rows at decode row counts, else torch's linear. wide_only: only where
     that is the faster one of the large projections (wq_b and wo_b, 84 MB each at the release's
     widths): at 33-64 rows the 128-row tiles (on 32-row tiles wo_b takes 32.8 against 29.0 us at 64
     rows), and up to 16 rows outputs wide enough to give every CU two 32-row tiles (wq_b
     1280 -> 32768, weights streamed: 18.7-19.8 us against the library's 21.6-22.4 us, 20.7-21.6
-    against 19.9-20.1 us at 24 and 32 rows; wo_b 8192 -> 5120 23.4-26.8 against 19.7-21.5 us)."""
+    against 19.9-20.1 us at 24 and 32 rows; wo_b 8192 -> 5120 23.4-26.8 against 19.7-21.5 us), where
+    the module call is the product alone."""
     if _decode_ok(lin, x):
         k, n = lin.weight.shape[1], lin.weight.shape[0]
         rows = x.numel() // k
         splits = _abi.linear_rows_splits(k, n, rows)
-        if not wide_only or (rows <= 16 and n >= 512 * 32) or _abi.linear_rows_wide(rows, k, n, splits):
+        few = rows <= 16 and n >= 512 * 32 and _only_the_product(lin, x)
+        if not wide_only or few or _abi.linear_rows_wide(rows, k, n, splits):
             return _abi.linear_rows(x.contiguous(), lin.weight, splits)
     return lin(x)
 

@@ -32,7 +32,7 @@ def test_wide_projection_at_decode_rows(gpu, rows):
     """A projection of at least 16,384 outputs, on either side of the row count where the library takes over."""
     from dsv41.layers import decode_linear
     g = torch.Generator(device="cuda").manual_seed(rows)
-    lin = torch.nn.Linear(192, 16384, bias=False, dtype=torch.bfloat16, device="cuda")
+    lin = torch.nn.Linear(192, 16384, bias=False, dtype=torch.bfloat16, device="cuda").requires_grad_(False)
     lin.weight.data.normal_(generator=g)
     x = torch.randn(rows, 192, generator=g, device="cuda").bfloat16()
     got = decode_linear(lin, x, wide_only=True)
@@ -40,3 +40,32 @@ def test_wide_projection_at_decode_rows(gpu, rows):
     # one rounding to bf16 (2^-8 of the value) of a float32 sum of 192 exact products
     sums = 192 * 2 ** -23 * (x.double().abs() @ lin.weight.double().abs().t())
     assert ((got.double() - want).abs() <= want.abs() * 2 ** -8 + sums).all()
+
+
+def test_wide_projection_keeps_what_the_module_call_does(gpu):
+    """At decode rows the kernel stands in for lin(x): hooks, gradients, a forward of the module's own and
+    tensors off 16-byte alignment still take the module."""
+    from dsv41.layers import decode_linear
+    lin = torch.nn.Linear(192, 16384, bias=False, dtype=torch.bfloat16, device="cuda").requires_grad_(False)
+    x = torch.randn(4, 192, device="cuda").bfloat16()
+    want = torch.nn.functional.linear(x, lin.weight)
+    calls = []
+    for register in (lin.register_forward_hook, lin.register_forward_pre_hook,
+                     torch.nn.modules.module.register_module_forward_hook):
+        handle = register(lambda *a: calls.append(a[0]))
+        decode_linear(lin, x, wide_only=True)
+        handle.remove()
+    assert calls == [lin] * 3
+    lin.forward = lambda t: torch.nn.functional.linear(t, lin.weight) * 2
+    assert torch.equal(decode_linear(lin, x, wide_only=True), want * 2)
+    del lin.forward
+
+    off = torch.empty(x.numel() + 1, dtype=x.dtype, device="cuda")[1:].view_as(x).copy_(x)
+    assert torch.equal(decode_linear(lin, off, wide_only=True), want)
+    lin.weight = torch.nn.Parameter(torch.empty(lin.weight.numel() + 1, dtype=x.dtype, device="cuda")[1:].view(16384, 192)
+                                    .copy_(lin.weight), requires_grad=False)
+    assert lin.weight.data_ptr() % 16 and torch.equal(decode_linear(lin, x, wide_only=True), want)
+
+    lin.requires_grad_(True)
+    decode_linear(lin, x.requires_grad_(), wide_only=True).float().sum().backward()
+    assert x.grad is not None and lin.weight.grad is not None
