@@ -69,3 +69,16 @@ def test_wide_projection_keeps_what_the_module_call_does(gpu):
     lin.requires_grad_(True)
     decode_linear(lin, x.requires_grad_(), wide_only=True).float().sum().backward()
     assert x.grad is not None and lin.weight.grad is not None
+
+
+@pytest.mark.parametrize("k,n,rows,own", [(1280, 32768, 16, True), (1280, 32768, 17, False), (4096, 16384, 1, True),
+                                          (4160, 16384, 16, False), (1280, 65536, 12, False)])
+def test_wide_projection_route(gpu, monkeypatch, k, n, rows, own):
+    """Weights of at most 2^26 values at up to 16 rows; the library streams larger ones at least as fast."""
+    from dsv41 import _abi, layers
+    calls = []
+    kernel = _abi.linear_rows
+    monkeypatch.setattr(_abi, "linear_rows", lambda *a: calls.append(1) or kernel(*a))
+    lin = torch.nn.Linear(k, n, bias=False, dtype=torch.bfloat16, device="cuda").requires_grad_(False)
+    layers.decode_linear(lin, torch.randn(rows, k, device="cuda").bfloat16(), wide_only=True)
+    assert bool(calls) == own
