@@ -62,14 +62,16 @@ def decode_linear(lin: torch.nn.Linear, x: torch.Tensor, wide_only: bool = False
     rows), and up to 16 rows outputs wide enough to give every CU two 32-row tiles (wq_b
     1280 -> 32768, weights streamed: 18.7-19.8 us against the library's 21.6-22.4 us, 20.7-21.6
     against 19.9-20.1 us at 24 and 32 rows; wo_b 8192 -> 5120 23.4-26.8 against 19.7-21.5 us), where
-    the module call is the product alone and the weight has at most 2^26 values: beyond, both stream it at
-    the same rate, the library a little faster at 12 and 16 rows (2048 -> 32768 34.1 against 34.6 us, but
-    4096 -> 32768 67.3-68.4 against 63.2 us, 1280 -> 65536 35.8-36.3 against 33.8 us)."""
+    the module call is the product alone. Outputs over 32,768, and over 24,576 with weights of 2^27 values
+    and more, stay with the library, which streams them as fast or faster (1280 -> 65536 35.8-36.3 against
+    33.8 us at 12 and 16 rows, 4096 -> 32768 65.3-68.4 against 62.5-63.3 us; but 8192 -> 16384 54.7-55.7
+    against 64.4-68.8 us, 2560 -> 32768 32.8-35.6 against 37.0-37.8 us)."""
     if _decode_ok(lin, x):
         k, n = lin.weight.shape[1], lin.weight.shape[0]
         rows = x.numel() // k
         splits = _abi.linear_rows_splits(k, n, rows)
-        few = rows <= 16 and n >= 512 * 32 and k * n <= 1 << 26 and _only_the_product(lin, x)
+        few = (rows <= 16 and 512 * 32 <= n <= 1 << 15 and (n <= 24576 or k * n < 1 << 27)
+               and _only_the_product(lin, x))
         if not wide_only or few or _abi.linear_rows_wide(rows, k, n, splits):
             return _abi.linear_rows(x.contiguous(), lin.weight, splits)
     return lin(x)
