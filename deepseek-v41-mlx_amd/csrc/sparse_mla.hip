@@ -1157,17 +1157,28 @@ struct MlaPlan {
 // stages at most kMaxList list entries.
 //
 // The two-role kernel (512 channels, whole 64-head groups) takes over past 128 of its workgroups: up to
-// there four splits per 32-head unit fill the chip evenly, past it two uneven rounds of long splits
-// would run. us, split lists -> two-role kernel, 64 heads:
+// there two to four splits per 32-head unit make one even round of the chip, past it two uneven rounds of
+// long splits would run. us, split lists -> two-role kernel, 64 heads:
 //   640 rows, bf16:    96 queries 36.8 -> 38.2, 130 59.5 -> 39.1, 200 77.9 -> 40.5, 240 76.1 -> 36.2
 //   640 rows, packed:  96 queries 52.1 -> 79.1, 130 123.0 -> 79.4, 200 162.5 -> 80.3
-//   2,176 rows, bf16:  128 queries 101.6 -> 79.3, 200 191.2 -> 80.0
+//   2,176 rows, bf16:  128 queries 101.6 -> 79.3 (still split), 200 191.2 -> 80.0
 //   window only, bf16: 128 tokens 20.2 -> 23.8, 130 queries 25.6 -> 23.7, 200 29.7 -> 24.3
-static MlaPlan plan_bf16(int64_t units, int heads, int list_max, int dim, bool two_role = true) {
+// Two kinds of list stay as they are for fewer queries. Of one step (32 entries), which need no combine:
+// 129 queries 12.2 -> 15.2, the first tokens of 129 sequences 14.0 -> 20.2, of 255 15.9 -> 21.0. And packed
+// rows of 256 entries and more whose two splits run the PAIR instance, up to three quarters of the chip:
+//   packed, 320 rows:  129 queries 45.2 -> 48.8, 185 47.0 -> 49.3, 220 52.4 -> 49.7
+//   packed, 448 rows:  129 queries 53.4 -> 61.2, 185 56.2 -> 61.5, 220 62.7 -> 62.0
+static MlaPlan plan_bf16(int64_t units, int heads, int list_max, int dim, int comp_format = kCompBf16,
+                         bool two_role = true) {
   MlaPlan p{};
   const int lm = list_max > 0 ? list_max : 1;
   const int hg32 = (heads + 31) / 32;
-  const bool roles = two_role && dim == 512 && heads % 64 == 0 && units * (heads / 64) > 128;
+  const int64_t wgs64 = units * (heads / 64);
+  const bool roles = two_role && dim == 512 && heads % 64 == 0 && wgs64 > 128 && lm > kStepRows;
+  if (roles && wgs64 <= 192 && (comp_format & kCompMask) == kCompFp4 && lm >= 8 * kStepRows) {
+    const MlaPlan split = plan_bf16(units, heads, list_max, dim, comp_format, false);
+    if (split.pair) return split;
+  }
   if ((units * hg32 >= 512 || roles) && lm <= kMaxList) {
     p.wide = heads > 32;
     p.hgroups = p.wide ? (heads + 63) / 64 : hg32;
@@ -1245,7 +1256,7 @@ static int run_mla(const char* what, MlaArgs a, int64_t units, int list_max, int
   if (dtype != DSV41_BF16) return set_error(DSV41_E_DTYPE, "%s: dtype %d not supported", what, dtype);
   DSV41_REQUIRE(bf16_dim_supported(a.dim), DSV41_E_SHAPE, "%s: bf16 path supports dim 64/128/256/512/576, got %d",
                 what, a.dim);
-  const MlaPlan p = plan_bf16(units, a.heads, list_max, a.dim);
+  const MlaPlan p = plan_bf16(units, a.heads, list_max, a.dim, comp_format);
   DSV41_REQUIRE(units * p.hgroups * p.splits < (1ll << 31), DSV41_E_ARG, "%s: too many workgroups", what);
   DSV41_REQUIRE(p.splits <= 64, DSV41_E_SHAPE, "%s: index list of %d entries is too long for the decode path", what,
                 list_max);
@@ -1293,9 +1304,9 @@ extern "C" size_t dsv41_sparse_mla_workspace_bytes(int32_t bsz, int32_t m, int32
   if (dtype != DSV41_BF16 || bsz <= 0 || m <= 0 || heads <= 0 || dim <= 0) return 0;
   const int64_t units = (int64_t)bsz * m;
   // What split lists take, also where the two-role kernel needs none: a buffer sized for 129-255 queries
-  // serves fewer, whose lists are split.
+  // serves fewer, whose lists are split, and packed rows, of which it takes fewer kinds.
   const size_t own = workspace_for(plan_bf16(units, heads, rows_per_query, dim), units, heads, dim);
-  const size_t split = workspace_for(plan_bf16(units, heads, rows_per_query, dim, false), units, heads, dim);
+  const size_t split = workspace_for(plan_bf16(units, heads, rows_per_query, dim, kCompBf16, false), units, heads, dim);
   return own > split ? own : split;
 }
 
