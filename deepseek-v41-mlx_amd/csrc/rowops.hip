@@ -319,13 +319,16 @@ static int launch_rows_ept(const RowArgs& a, hipStream_t stream, const char* wha
   return check_launch(what);
 }
 
-// 8 elements per thread, unless a fused norm would need more than 64 lanes for one row. A prompt's index
-// queries (a rope and no norm) take 16 once 8 would make 2^20 threads: the row's position costs three
-// integer divisions per thread (us at 8 | 16 | 32 elements: 8,192 x 64 heads 79.8 | 70.5 | 66.3, as
-// MXFP4 69.4 | 55.3 | 49.0; 2,048 x 32 heads 17.8 | 16.3 | 17.4).
+// 8 elements per thread, unless a fused norm would need more than 64 lanes for one row. Rope without a norm
+// on many bf16 rows (a prompt's index queries, its attention output, an fp8 cache write) takes 16 once 8
+// would make 2^20 threads: the row's position costs three integer divisions per thread. us at 8 | 16 | 32
+// elements: index queries of 8,192 x 64 heads 79.8 | 70.5 | 66.3, as MXFP4 69.4 | 55.3 | 49.0, of 2,048 x 32
+// heads 17.8 | 16.3 | 17.4; at 8 | 16: rope_tail of 4,096 x 64 x 512 107.4 | 94.1, of 16,384 x 512 10.4 | 9.1,
+// comp_write_fp8 of 16,384 rows 13.2 | 11.5. float32 rows stay at 8 (rope_tail of 16,384 x 512 12.9 | 19.1, of
+// 4,096 x 64 x 512 184 | 222: the lanes of one load would lie 64 bytes apart).
 template <typename T, bool NORM, bool ROPE, int FQ, int BLK>
 static int launch_rows(const RowArgs& a, hipStream_t stream, const char* what) {
-  if constexpr (ROPE && !NORM && BLK == 32)
+  if constexpr (ROPE && !NORM && BLK == 32 && sizeof(T) == 2)
     if (a.rows * a.cpr * 4 >= (int64_t)1 << 20) return launch_rows_ept<T, NORM, ROPE, FQ, BLK, 16>(a, stream, what);
   if (!NORM || a.cpr * 4 <= 64) return launch_rows_ept<T, NORM, ROPE, FQ, BLK, 8>(a, stream, what);
   return launch_rows_ept<T, NORM, ROPE, FQ, BLK, 32>(a, stream, what);
