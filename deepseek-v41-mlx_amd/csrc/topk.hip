@@ -672,12 +672,20 @@ constexpr int kStripeMax = 32 * kSelThreads;   // entries of the largest stripe 
 // on scores already in cache (17.5-19.3 against 19.4-20.2 us), but inside a decode step, reading
 // the scores the scoring kernel has just written, the two stages spread that read over 8
 // workgroups per row and win: the 40-layer fp8 step took 1.163-1.166 ms against 1.190-1.195 ms.
-static int64_t stripe_from(int nb) { return nb <= 16 * kSelThreads ? 512 : (nb <= kStripeMax ? 64 : 128); }
+//
+// Rows over 24,576 scores whose two stages have short lists (k up to 1,024) win for a few rows more: 64 rows
+// of 32,768 scores, two stages -> stripe, top-128 13.1 -> 14.8 us, top-512 15.5 -> 15.6, top-2,048 23.0 ->
+// 16.0; 72 rows of 28,000, top-128 13.1 -> 14.8; 80 rows of 32,768, top-128 15.8 -> 14.8.
+static int64_t stripe_from(int nb, int k) {
+  if (nb <= 16 * kSelThreads) return 512;
+  if (nb <= kStripeMax) return nb <= 24 * kSelThreads || k > 1024 ? 64 : 80;
+  return 128;
+}
 
 static TopkPlan topk_plan(int64_t rows, int nb, int k, bool allow_two_stage) {
   TopkPlan p{false, 0, 0};
   if (k >= nb) return p;                           // everything is selected
-  const bool many = rows >= stripe_from(nb);
+  const bool many = rows >= stripe_from(nb, k);
   if (nb <= kStripeMax) {
     p.stripe = many;
     if (p.stripe) return p;
@@ -817,7 +825,7 @@ extern "C" size_t dsv41_topk_workspace_bytes(int64_t rows, int32_t nb, int32_t t
     const TopkPlan p = topk_plan(r, nb, k, true);
     return p.chunks ? topk_ws_bytes(r, p.chunks, k) : (size_t)0;
   };
-  const int64_t few = stripe_from(nb) - 1;
+  const int64_t few = stripe_from(nb, k) - 1;
   const size_t own = bytes(rows), less = rows > few ? bytes(few) : 0;
   return own > less ? own : less;
 }

@@ -29,6 +29,7 @@ def _scores(rows, nb, kind):
     (512, 2, 1), (513, 65, 64), (512, 2048, 512), (600, 2049, 2048), (512, 4096, 1), (512, 4097, 512),
     (512, 6145, 6144), (512, 8193, 777), (530, 10240, 2048), (512, 10241, 512), (512, 12289, 512), (512, 16384, 1024),
     (64, 16385, 512), (70, 20481, 2048), (64, 24577, 512), (64, 32768, 4096),
+    (79, 24577, 1024), (80, 24577, 1024), (64, 32768, 1025),
     (128, 32769, 512),                   # two chunks, the second a little shorter
     (130, 65536, 2048), (128, 65600, 512),
     (128, 98305, 4096),                  # four chunks

@@ -13,6 +13,14 @@ def test_topk_workspace_never_falls_with_rows(nb, k):
     assert sizes == sorted(sizes)
 
 
+def test_topk_rows_from_which_one_workgroup_selects_a_row():
+    """The last row count that still takes two stages is the one whose workspace is the largest."""
+    from dsv41 import _abi
+    for nb, k, last in [(24576, 512, 63), (24577, 1024, 79), (32768, 64, 79), (32768, 1025, 63), (40000, 512, 127)]:
+        sizes = [_abi.topk_workspace_bytes(r, nb, k) for r in range(1, 128)]
+        assert sizes.index(max(sizes)) + 1 == last, (nb, k)
+
+
 @pytest.mark.parametrize("heads,most", [(64, 255), (64, 200), (64, 130), (128, 127), (128, 70)])
 @pytest.mark.parametrize("rows", [128, 640, 2176])
 def test_attention_workspace_of_a_batch_serves_its_half(heads, most, rows):
