@@ -552,11 +552,13 @@ __global__ __launch_bounds__(kSelThreads) void topk_kernel(const float* __restri
 }
 
 constexpr int kMaxCandBlocks = 8192;
-// Rows from which candidate blocks of 8 scores run on topk_stripe_kernel, us candidate_kernel -> stripe
-// (rows of 32,768 scores, 2,048 blocks kept): 64 rows 11.2 -> 10.3, 384 rows 21.8 ->
-// 15.9, 2,048 rows 99.0 -> 63.6; 1,400 x 22,804 417 us with byte stores and scalar reads of the rows
-// that are not 16-byte pieces, 52 us with element-aligned ones, 33.6 us on the stripe kernel.
-constexpr int64_t kCandStripeRows = 64;
+// Rows from which candidate blocks of 8 scores run on topk_stripe_kernel, us candidate_kernel -> stripe.
+// 32,768 scores, 2,048 blocks kept: 64 rows 11.2 -> 10.3, 384 rows 21.8 -> 15.9, 2,048 rows 99.0 -> 63.6;
+// 1,400 x 22,804 417 us with byte stores and scalar reads of the rows that are not 16-byte pieces, 52 us with
+// element-aligned ones, 33.6 us on the stripe kernel. Up to 1,024 blocks the register kernel's one short
+// pass wins until the rows fill the chip more than once (4,096 scores, 64 blocks kept: 64 rows 5.9 -> 6.4,
+// 256 rows 6.6 -> 7.1, 384 rows 8.1 -> 7.3, 512 rows 8.7 -> 7.5).
+static int64_t cand_stripe_from(int nblk) { return nblk > kSelThreads ? 64 : 384; }
 
 // select_candidate_blocks on the register core: thread t holds the maxima of blocks t*J ..
 // t*J+J-1 as order keys (the pinned block (lens-1)/bs as +inf); the best min(topk_blocks, nblk)
@@ -851,7 +853,7 @@ extern "C" int dsv41_candidate_blocks(const float* scores, uint8_t* keep, int64_
   const int nblk = (nb + block_size - 1) / block_size;
   // a whole block of NaNs counts as NaN where the rows are 16-byte pieces, else as -inf
   const int nan_blocks = nb % 8 == 0 && aligned16(scores) && (reinterpret_cast<uintptr_t>(keep) & 7u) == 0 ? 1 : 0;
-  if (block_size == 8 && rows >= kCandStripeRows && topk_blocks > 0 && topk_blocks < nblk) {
+  if (block_size == 8 && rows >= cand_stripe_from(nblk) && topk_blocks > 0 && topk_blocks < nblk) {
     launch_stripe<kStripeBlocks>(nblk, (unsigned)rows, scores, nullptr, n, nb, topk_blocks, start_pos, ratio, 0, 1, nb,
                                  nullptr, nullptr, keep, lens, nan_blocks, stream);
     return check_launch(what);

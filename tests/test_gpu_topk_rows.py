@@ -63,6 +63,7 @@ def test_rows_down_to_infinity_and_below(gpu, nb, k, inf):
 @pytest.mark.parametrize("rows,nb,kb", [
     (512, 9, 1), (512, 4097, 300), (513, 16384, 2047), (520, 16385, 2048), (515, 22804, 2048),
     (512, 32776, 4096), (512, 65536, 1),
+    (64, 8193, 700), (383, 8192, 64), (384, 8192, 64),   # either side of 1,024 blocks and of 384 rows
 ])
 @pytest.mark.parametrize("kind", ["normal", "ties", "masked", "odd"])
 def test_candidate_rows_equal_few_rows(gpu, rows, nb, kb, kind):
