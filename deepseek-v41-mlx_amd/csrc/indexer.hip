@@ -930,10 +930,33 @@ __global__ __launch_bounds__(64 * kPfQueries / NQ, NQ == 1 ? 4 : 3) void indexer
   }
 }
 
-// Key rows per prefill workgroup: kPfRows, halved down to 256 while fewer than 512 workgroups (two
-// per CU) would run: a chunk of a few dozen queries leaves most of the chip idle otherwise (64 heads,
-// 10,240 keys: 8 queries 54.5 -> 12.5 us, 64 queries 55.9 -> 19.2 us, 512 queries 98.9 -> 80.3 us).
-static int prefill_rows(int64_t groups, int nb) {
+// Key rows per prefill workgroup, in whole ring chunks: even ranges of the least time for `groups` workgroups
+// per range, nq queries per wave. In units of a chunk of a workgroup alone on its CU (1.64 us at 64 heads,
+// 1.08 at 32, 0.73 at 16) c chunks were measured to take c + 1.5 there, 1.6 c + 3 (nq 2) and 1.75 c + 3 (nq 1)
+// for two on a CU and 1.9 c + 4.5 for three (nq 2); more workgroups come in rounds. Halving the range until
+// two per CU ran left short last ranges behind and repeated fixed costs: us, 64 heads, one range | powers of
+// two | even ranges: 2,000 queries x 600 keys 25.1 | 29.9 | 24.2, 2,000 x 1,100 38.9 | 49.9 | 39.7, 1,500 x
+// 1,500 45.9 | 44.9 | 40.2, 512 x 8,192 (ranges of 2,048) 62.9 | 59.8 | 59.5, 16 x 36,864 56.1 | 19.4 | 15.1.
+static int prefill_rows(int64_t groups, int nb, int nq) {
+  const int chunks = (nb + kPfChunk - 1) / kPfChunk;
+  int best = 4;
+  double least = 1e30;
+  for (int c = min(kPfRows / kPfChunk, chunks); c >= min(4, chunks); --c) {
+    const double lone = c + 1.5, two = (nq == 2 ? 1.6 : 1.75) * c + 3, three = 1.9 * c + 4.5;
+    const int64_t w = groups * ((chunks + c - 1) / c), round = nq == 2 ? 768 : 512, rest = w % round;
+    const double t = (double)(w / round) * (nq == 2 ? three : two) +
+                     (rest == 0 ? 0.0 : rest <= 256 ? lone : rest <= 512 ? two : three);
+    if (t < least) {
+      least = t;
+      best = c;
+    }
+  }
+  return best * kPfChunk;
+}
+
+// The same for the MXFP4 chunk kernel, whose workgroups take 256 rows at a time: kPfRows, halved down to 256
+// while fewer than 512 workgroups (two per CU) would run.
+static int mx_chunk_rows(int64_t groups, int nb) {
   int r = kPfRows;
   while (r > 256 && groups * ((nb + r - 1) / r) < 512) r /= 2;
   return r;
@@ -1029,17 +1052,20 @@ extern "C" int dsv41_indexer_score(const void* q, const void* w_raw, float w_sca
   if (n >= 8 && dim == 128 && (heads == 64 || heads == 32 || heads == 16) &&
       (int64_t)bsz * ((n + 7) / 8) < 65536) {
     const int64_t groups = (int64_t)bsz * ((n + kPfQueries - 1) / kPfQueries);
-    const int rows = prefill_rows(groups, nb);
+    // short caches of 32 heads are all fixed cost, which two queries per wave make longer (1,600 queries x 300
+    // keys 10.0 us with one, 10.6 with two)
+    const int nq = candidates || heads > 32 || (heads == 32 && nb <= 384) ? 1 : 2;
+    const int rows = prefill_rows(groups, nb, nq);
     const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
     const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_PF_CASE(HT_, NQ_, CAND_)                                                                      \
-    if (heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                             \
+    if (heads == HT_ * 16 && nq == NQ_ && (candidates != nullptr) == CAND_) {                                             \
       hipLaunchKernelGGL((indexer_prefill_kernel<HT_, NQ_, CAND_, false>), pgrid, dim3(64 * kPfQueries / NQ_), 0, \
                          stream, (const bf16_t*)q, (const bf16_t*)w_raw, w_scale, index_k, k_bstride, nullptr, \
                          0, 0, candidates, scores, n, nb, start_pos, ratio, rows, cvec);                      \
       return check_launch(what);                                                                             \
     }
-    DSV41_PF_CASE(4, 1, false) DSV41_PF_CASE(2, 2, false) DSV41_PF_CASE(1, 2, false)
+    DSV41_PF_CASE(4, 1, false) DSV41_PF_CASE(2, 2, false) DSV41_PF_CASE(2, 1, false) DSV41_PF_CASE(1, 2, false)
     DSV41_PF_CASE(4, 1, true) DSV41_PF_CASE(2, 1, true) DSV41_PF_CASE(1, 1, true)
 #undef DSV41_PF_CASE
   }
@@ -1126,7 +1152,7 @@ extern "C" int dsv41_indexer_score_fp8(const void* q, const void* w_raw, float w
   if ((int64_t)bsz * n == 0 || nb == 0) return 0;
   if (n >= 8 && (heads == 64 || heads == 32 || heads == 16)) {
     const int64_t groups = (int64_t)bsz * ((n + kPfQueries - 1) / kPfQueries);
-    const int rows = prefill_rows(groups, nb);
+    const int rows = prefill_rows(groups, nb, !candidates && heads <= 32 ? 2 : 1);
     const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
     const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_PF8_CASE(HT_, NQ_, CAND_)                                                                       \
@@ -1197,7 +1223,7 @@ static int mx_score_entry(const char* what, bool kf8, const uint8_t* q_codes, co
   if (!kf8 && n >= 8 && (heads == 64 || heads == 32 || heads == 16)) {
     const int nq = kMxChunkTiles * 16 / heads;
     const int64_t groups = (int64_t)bsz * ((n + nq - 1) / nq);
-    const int rows = prefill_rows(groups, nb);
+    const int rows = mx_chunk_rows(groups, nb);
     const dim3 cgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_MXCHUNK_CASE(HT_, CAND_)                                                                        \
     if (heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                              \

@@ -124,3 +124,30 @@ def test_fp8_chunk_scores_equal_per_query(gpu, b, n, heads, nb, start, ratio, rb
         rows.append(_abi.indexer_score_fp8(q[:, s:s + 1].contiguous(), w[:, s:s + 1].contiguous(), 0.07, codes, scales,
                                            rb, nb, start + s, ratio, c))
     assert torch.equal(got, torch.cat(rows, 1))
+
+
+# (queries, keys): ranges of 10 chunks in one piece; of 9 and 9; of 300 keys with one query per wave at 32
+# heads; of many even pieces with a short last one; masks read by vectors (1,104, 3,008) and by bytes
+RANGES = [(1700, 600), (1501, 1100), (1999, 300), (301, 3008), (430, 1104), (77, 16500)]
+
+
+@pytest.mark.parametrize("n,nb", RANGES)
+@pytest.mark.parametrize("heads", [16, 32, 64])
+@pytest.mark.parametrize("fmt,keep", [("bf16", None), ("bf16", 0.3), ("fp8", None), ("fp8", 0.3)])
+def test_chunk_ranges_equal_few_queries(gpu, fmt, keep, heads, n, nb):
+    from dsv41 import _abi
+    g, q, w, k = _inputs(1, n, heads, nb, nb + n)
+    codes = k.to(torch.float8_e4m3fn).view(torch.uint8)
+    scales = torch.randint(118, 132, (1, (nb + 31) // 32, 4), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    cand = None if keep is None else torch.rand(1, n, nb, generator=g, device="cuda").lt(keep).contiguous()
+    start = max(nb - n // 2, 0)          # the causal edge runs through the last keys
+
+    def run(lo, hi):
+        c = None if cand is None else cand[:, lo:hi].contiguous()
+        a = (q[:, lo:hi].contiguous(), w[:, lo:hi].contiguous(), 0.07)
+        if fmt == "fp8":
+            return _abi.indexer_score_fp8(*a, codes, scales, 32, nb, start + lo, 1, c)
+        return _abi.indexer_score(*a, k, start + lo, 1, c)
+
+    few = torch.cat([run(lo, min(lo + 7, n)) for lo in range(0, n, 7)], 1)
+    assert torch.equal(run(0, n), few)
