@@ -937,7 +937,7 @@ __global__ __launch_bounds__(64 * kPfQueries / NQ, NQ == 1 ? 4 : 3) void indexer
 // two per CU ran left short last ranges behind and repeated fixed costs: us, 64 heads, one range | powers of
 // two | even ranges: 2,000 queries x 600 keys 25.1 | 29.9 | 24.2, 2,000 x 1,100 38.9 | 49.9 | 39.7, 1,500 x
 // 1,500 45.9 | 44.9 | 40.2, 512 x 8,192 (ranges of 2,048) 62.9 | 59.8 | 59.5, 16 x 36,864 56.1 | 19.4 | 15.1.
-static int prefill_rows(int64_t groups, int nb, int nq) {
+static int prefill_rows(int64_t groups, int nb, int nq, double* time) {
   const int chunks = (nb + kPfChunk - 1) / kPfChunk;
   int best = 4;
   double least = 1e30;
@@ -951,6 +951,7 @@ static int prefill_rows(int64_t groups, int nb, int nq) {
       best = c;
     }
   }
+  *time = least;
   return best * kPfChunk;
 }
 
@@ -1021,6 +1022,46 @@ static dim3 idx_grid(int64_t rows_total, int nb, int bn, int* rows_per_wg) {
   return dim3((unsigned)((nb + r - 1) / r), (unsigned)bn);
 }
 
+// Chunks of 8 and more queries on few scores are mostly a chunk kernel's fixed cost (its queries, mask and
+// first keys), and a workgroup per query and key range is done sooner: 16 masked queries x 2,048 bf16 keys,
+// 64 heads, 6.4 us against 13.5. Which is, is read off the times of both kernels over 8 to 500 queries,
+// 100 to 36,864 keys and 1 to 16 sequences (within 1 % of the better one on average); a tie of 5 % goes to
+// the one-query kernel, except over MXFP4. us:
+//   one-query kernels: base + rounds of 256 workgroups x (step + rows x key rows / 1,024), + far x 10^6 scores
+//     where the batch's keys outgrow an XCD's L2
+//   indexer_prefill_kernel: base + unit x prefill_rows' time
+//   indexer_mx_chunk_kernel: base + rounds of 256 workgroups x (step + rows x key rows / 1,024)
+// each for 16, 32 and 64 heads. Unmasked bf16 chunks always gain (16 queries x 2,048 keys, 64 heads 12.7 us).
+constexpr double kPlainOneQuery = 1.6;   // the register kernel, where the staged one's alignment is missing
+struct OneQueryUs {
+  double base, step, rows, far;
+};
+struct ChunkUs {
+  double base, unit;
+};
+struct MxChunkUs {
+  double base, step, rows;
+};
+constexpr OneQueryUs kOneQueryBf16[3] = {{3.5, 0.67, 3.2, 6.7}, {3.4, 0.86, 3.4, 6.7}, {3.3, 1.3, 4.1, 6.3}};
+constexpr OneQueryUs kOneQueryFp8[3] = {{3.9, 0.62, 2.65, 2.4}, {3.8, 0.82, 3.1, 2.2}, {3.8, 1.13, 4.1, 2.3}};
+constexpr OneQueryUs kOneQueryMx[3] = {{4.0, 0.42, 1.25, 0.7}, {4.0, 0.63, 1.45, 0.85}, {4.0, 1.05, 2.0, 0.7}};
+constexpr ChunkUs kChunkBf16Masked[3] = {{4.3, 0.68}, {4.2, 1.03}, {4.6, 1.79}};
+constexpr ChunkUs kChunkFp8[3] = {{3.1, 0.77}, {2.6, 1.28}, {3.0, 2.06}};
+constexpr ChunkUs kChunkFp8Masked[3] = {{4.5, 0.69}, {4.6, 1.02}, {5.3, 1.75}};
+constexpr MxChunkUs kChunkMx[3] = {{5.4, 0.33, 4.5}, {4.9, 0.42, 3.7}, {4.65, 0.44, 3.2}};
+
+static int head_class(int heads) { return heads == 16 ? 0 : (heads == 32 ? 1 : 2); }
+
+static double rounds_of(int64_t workgroups) { return (double)((workgroups + 255) / 256); }
+
+static double one_query_us(const OneQueryUs& t, int bsz, int n, int nb, int key_bytes) {
+  int rows = 0;
+  const dim3 grid = idx_grid((int64_t)nb * bsz * n, nb, bsz * n, &rows);
+  const bool far = (int64_t)bsz * nb * key_bytes >= 7 << 19;   // 3.5 of 4 MB
+  return t.base + rounds_of((int64_t)grid.x * grid.y) * (t.step + t.rows * min(rows, nb) / 1024.0) +
+         (far ? t.far * 1e-6 * bsz * n * nb : 0.0);
+}
+
 }  // namespace dsv41
 
 using namespace dsv41;
@@ -1055,11 +1096,16 @@ extern "C" int dsv41_indexer_score(const void* q, const void* w_raw, float w_sca
     // short caches of 32 heads are all fixed cost, which two queries per wave make longer (1,600 queries x 300
     // keys 10.0 us with one, 10.6 with two)
     const int nq = candidates || heads > 32 || (heads == 32 && nb <= 384) ? 1 : 2;
-    const int rows = prefill_rows(groups, nb, nq);
+    double time = 0.0;
+    const int rows = prefill_rows(groups, nb, nq, &time);
+    const int hc = head_class(heads);
+    const ChunkUs& t = kChunkBf16Masked[hc];
+    const bool gains = !candidates || t.base + t.unit * time < one_query_us(kOneQueryBf16[hc], bsz, n, nb, 2 * dim) *
+                                                                   (aligned16(w_raw) ? 0.95 : kPlainOneQuery);
     const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
     const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_PF_CASE(HT_, NQ_, CAND_)                                                                      \
-    if (heads == HT_ * 16 && nq == NQ_ && (candidates != nullptr) == CAND_) {                                             \
+    if (gains && heads == HT_ * 16 && nq == NQ_ && (candidates != nullptr) == CAND_) {                                           \
       hipLaunchKernelGGL((indexer_prefill_kernel<HT_, NQ_, CAND_, false>), pgrid, dim3(64 * kPfQueries / NQ_), 0, \
                          stream, (const bf16_t*)q, (const bf16_t*)w_raw, w_scale, index_k, k_bstride, nullptr, \
                          0, 0, candidates, scores, n, nb, start_pos, ratio, rows, cvec);                      \
@@ -1152,11 +1198,17 @@ extern "C" int dsv41_indexer_score_fp8(const void* q, const void* w_raw, float w
   if ((int64_t)bsz * n == 0 || nb == 0) return 0;
   if (n >= 8 && (heads == 64 || heads == 32 || heads == 16)) {
     const int64_t groups = (int64_t)bsz * ((n + kPfQueries - 1) / kPfQueries);
-    const int rows = prefill_rows(groups, nb, !candidates && heads <= 32 ? 2 : 1);
+    double time = 0.0;
+    const int rows = prefill_rows(groups, nb, !candidates && heads <= 32 ? 2 : 1, &time);
+    const int hc = head_class(heads);
+    const ChunkUs& t = candidates ? kChunkFp8Masked[hc] : kChunkFp8[hc];
+    const bool staged = aligned16(w_raw) && aligned16(k_scale) && ks_bstride % 16 == 0;
+    const bool gains = t.base + t.unit * time <
+                       one_query_us(kOneQueryFp8[hc], bsz, n, nb, dim) * (staged ? 0.95 : kPlainOneQuery);
     const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
     const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_PF8_CASE(HT_, NQ_, CAND_)                                                                       \
-    if (heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                              \
+    if (gains && heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                     \
       hipLaunchKernelGGL((indexer_prefill_kernel<HT_, NQ_, CAND_, true>), pgrid, dim3(64 * kPfQueries / NQ_), 0, \
                          stream, (const bf16_t*)q, (const bf16_t*)w_raw, w_scale, index_k, k_bstride, k_scale, \
                          ks_bstride, ks_rb == 32 ? 5 : 0, candidates, scores, n, nb, start_pos, ratio, rows, cvec); \
@@ -1224,9 +1276,13 @@ static int mx_score_entry(const char* what, bool kf8, const uint8_t* q_codes, co
     const int nq = kMxChunkTiles * 16 / heads;
     const int64_t groups = (int64_t)bsz * ((n + nq - 1) / nq);
     const int rows = mx_chunk_rows(groups, nb);
+    const int hc = head_class(heads);
+    const MxChunkUs& t = kChunkMx[hc];
+    const bool gains = t.base + rounds_of(groups * ((nb + rows - 1) / rows)) * (t.step + t.rows * min(rows, nb) / 1024.0) <
+                       one_query_us(kOneQueryMx[hc], bsz, n, nb, dim / 2);
     const dim3 cgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_MXCHUNK_CASE(HT_, CAND_)                                                                        \
-    if (heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                              \
+    if (gains && heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                     \
       hipLaunchKernelGGL((indexer_mx_chunk_kernel<HT_, CAND_>), cgrid, dim3(kMxChunkThreads), 0, stream, q_codes, \
                          q_scales, (const bf16_t*)w_raw, w_scale, k_codes, kc_bstride, k_scales, ks_bstride,  \
                          candidates, scores, n, nb, start_pos, ratio, rows);                                  \

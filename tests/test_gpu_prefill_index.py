@@ -126,28 +126,36 @@ def test_fp8_chunk_scores_equal_per_query(gpu, b, n, heads, nb, start, ratio, rb
     assert torch.equal(got, torch.cat(rows, 1))
 
 
-# (queries, keys): ranges of 10 chunks in one piece; of 9 and 9; of 300 keys with one query per wave at 32
-# heads; of many even pieces with a short last one; masks read by vectors (1,104, 3,008) and by bytes
-RANGES = [(1700, 600), (1501, 1100), (1999, 300), (301, 3008), (430, 1104), (77, 16500)]
+# (queries, keys, start, ratio). Ranges: of 10 chunks in one piece; of 9 and 9; of 300 keys with one query per
+# wave at 32 heads; of many even pieces with a short last one; masks read by vectors (1,104, 3,008) and by bytes.
+RANGES = [(1700, 600, 0, 1), (1501, 1100, 350, 1), (1999, 300, 0, 1), (301, 3008, 2858, 1), (430, 1104, 889, 1),
+          (77, 16500, 16462, 1)]
+# Edges, over enough scores for the chunk kernels: one key, which the first query does not see at ratio 2;
+# partial last query groups; a partial chunk with the causal edge inside; queries before and after the last key.
+EDGES = [(3000, 1, 0, 2), (2001, 63, 40, 1), (1999, 64, 60, 1), (999, 2047, 7500, 4), (601, 4101, 16100, 4)]
 
 
-@pytest.mark.parametrize("n,nb", RANGES)
+@pytest.mark.parametrize("n,nb,start,ratio,keep", [(*c, keep) for keep in (None, 0.3) for c in RANGES + EDGES] +
+                         [(*c, 0.0) for c in EDGES[:3]])
 @pytest.mark.parametrize("heads", [16, 32, 64])
-@pytest.mark.parametrize("fmt,keep", [("bf16", None), ("bf16", 0.3), ("fp8", None), ("fp8", 0.3)])
-def test_chunk_ranges_equal_few_queries(gpu, fmt, keep, heads, n, nb):
+@pytest.mark.parametrize("fmt", ["bf16", "fp8", "mxfp4"])
+def test_chunk_scores_equal_few_queries(gpu, fmt, keep, heads, n, nb, start, ratio):
     from dsv41 import _abi
     g, q, w, k = _inputs(1, n, heads, nb, nb + n)
+    ints = lambda lo, hi, *s: torch.randint(lo, hi, s, generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
     codes = k.to(torch.float8_e4m3fn).view(torch.uint8)
-    scales = torch.randint(118, 132, (1, (nb + 31) // 32, 4), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    scales = ints(118, 132, 1, (nb + 31) // 32, 4)
+    q4, qs, k4, ks = ints(0, 256, 1, n, heads, 64), ints(118, 132, 1, n, heads, 4), ints(0, 256, 1, nb, 64), ints(118, 132, 1, nb, 4)
     cand = None if keep is None else torch.rand(1, n, nb, generator=g, device="cuda").lt(keep).contiguous()
-    start = max(nb - n // 2, 0)          # the causal edge runs through the last keys
 
     def run(lo, hi):
-        c = None if cand is None else cand[:, lo:hi].contiguous()
-        a = (q[:, lo:hi].contiguous(), w[:, lo:hi].contiguous(), 0.07)
+        part = lambda t: t[:, lo:hi].contiguous()
+        c, ws = None if cand is None else part(cand), (part(w), 0.07)
+        if fmt == "mxfp4":
+            return _abi.indexer_score_mxfp4((part(q4), part(qs)), *ws, k4, ks, nb, start + lo, ratio, c)
         if fmt == "fp8":
-            return _abi.indexer_score_fp8(*a, codes, scales, 32, nb, start + lo, 1, c)
-        return _abi.indexer_score(*a, k, start + lo, 1, c)
+            return _abi.indexer_score_fp8(part(q), *ws, codes, scales, 32, nb, start + lo, ratio, c)
+        return _abi.indexer_score(part(q), *ws, k, start + lo, ratio, c)
 
     few = torch.cat([run(lo, min(lo + 7, n)) for lo in range(0, n, 7)], 1)
     assert torch.equal(run(0, n), few)
