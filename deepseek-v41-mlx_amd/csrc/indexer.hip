@@ -930,22 +930,48 @@ __global__ __launch_bounds__(64 * kPfQueries / NQ, NQ == 1 ? 4 : 3) void indexer
   }
 }
 
-// Key rows per prefill workgroup, in whole ring chunks: even ranges of the least time for `groups` workgroups
-// per range, nq queries per wave. In units of a chunk of a workgroup alone on its CU (1.64 us at 64 heads,
-// 1.08 at 32, 0.73 at 16) c chunks were measured to take c + 1.5 there, 1.6 c + 3 (nq 2) and 1.75 c + 3 (nq 1)
-// for two on a CU and 1.9 c + 4.5 for three (nq 2); more workgroups come in rounds. Halving the range until
-// two per CU ran left short last ranges behind and repeated fixed costs: us, 64 heads, one range | powers of
-// two | even ranges: 2,000 queries x 600 keys 25.1 | 29.9 | 24.2, 2,000 x 1,100 38.9 | 49.9 | 39.7, 1,500 x
-// 1,500 45.9 | 44.9 | 40.2, 512 x 8,192 (ranges of 2,048) 62.9 | 59.8 | 59.5, 16 x 36,864 56.1 | 19.4 | 15.1.
-static int prefill_rows(int64_t groups, int nb, int nq, double* time) {
+// Keys that a chunk's first and last queries see, of nb: the workgroups past them only store -inf.
+struct Seen {
+  double first, last, mean;
+};
+static Seen seen_keys(int start_pos, int n, int ratio, int nb) {
+  Seen s;
+  s.first = fmin((double)nb, (double)(start_pos + 1) / ratio);
+  s.last = fmin((double)nb, (double)(start_pos + n) / ratio);
+  s.mean = 0.5 * (s.first + s.last);
+  return s;
+}
+// Of `ranges` ranges of `rows` keys for each of `groups` query groups, those that some query sees into: with
+// the visible keys spread over a range and more, half a range past their mean.
+static int64_t workgroups_seen(int64_t groups, double rows, int ranges, const Seen& s) {
+  const double per = s.last - s.first < rows ? ceil(s.last / rows) : s.mean / rows + 0.5;
+  return (int64_t)ceil((double)groups * fmin((double)ranges, per));
+}
+
+// Key rows per prefill workgroup, in whole ring chunks: even ranges of the least time for `groups` query groups,
+// nq queries per wave. Times in units of a chunk of a workgroup alone on its CU (1.64 us at 64 heads, 1.08 at 32,
+// 0.73 at 16). Where all queries see about the same keys, workgroups come in rounds: c chunks were measured to
+// take c + 1.5 alone on a CU, 1.6 c + 3 (nq 2) and 1.75 c + 3 (nq 1) for two on it and 1.9 c + 4.5 for three
+// (nq 2). Where the causal edge runs through the keys, ranges are of many lengths and workgroups fill in for
+// one another: the chip does 256 x 1.5 units at once, and half a workgroup's time passes until the last is
+// done. Over 248 sizes (64 to 8,192 queries, 600 to 32,768 keys, with and without a mask, bf16 and fp8 keys)
+// this loses 2.6 % on average against the best of 17 lengths; halving the range until two workgroups per CU
+// ran lost 10 %, as it left short last ranges behind and repeated fixed costs. us, 64 heads, one range | powers
+// of two | these: 2,000 queries x 600 keys 25.1 | 29.9 | 24.2, 2,000 x 1,100 38.9 | 49.9 | 39.7, 1,500 x 1,500
+// 45.9 | 44.9 | 40.2, 512 x 8,192 (ranges of 2,048) 62.9 | 59.8 | 59.5, 16 x 36,864 56.1 | 19.4 | 15.1.
+static int prefill_rows(int64_t groups, int nb, const Seen& seen, int nq, double* time) {
   const int chunks = (nb + kPfChunk - 1) / kPfChunk;
+  const bool same = seen.last - seen.first <= fmax(seen.last / 8, (double)kPfChunk);
+  const double all = (double)groups * (seen.mean / kPfChunk + 0.5);
   int best = 4;
   double least = 1e30;
   for (int c = min(kPfRows / kPfChunk, chunks); c >= min(4, chunks); --c) {
+    const int64_t w = workgroups_seen(groups, (double)kPfChunk * c, (chunks + c - 1) / c, seen);
     const double lone = c + 1.5, two = (nq == 2 ? 1.6 : 1.75) * c + 3, three = 1.9 * c + 4.5;
-    const int64_t w = groups * ((chunks + c - 1) / c), round = nq == 2 ? 768 : 512, rest = w % round;
-    const double t = (double)(w / round) * (nq == 2 ? three : two) +
-                     (rest == 0 ? 0.0 : rest <= 256 ? lone : rest <= 512 ? two : three);
+    const int64_t round = nq == 2 ? 768 : 512, rest = w % round;
+    double t = (double)(w / round) * (nq == 2 ? three : two) +
+               (rest == 0 ? 0.0 : rest <= 256 ? lone : rest <= 512 ? two : three);
+    if (!same) t = fmax(lone, (all + 1.5 * w) / 384.0 + 0.5 * lone);
     if (t < least) {
       least = t;
       best = c;
@@ -1054,12 +1080,13 @@ static int head_class(int heads) { return heads == 16 ? 0 : (heads == 32 ? 1 : 2
 
 static double rounds_of(int64_t workgroups) { return (double)((workgroups + 255) / 256); }
 
-static double one_query_us(const OneQueryUs& t, int bsz, int n, int nb, int key_bytes) {
+static double one_query_us(const OneQueryUs& t, int bsz, int n, int nb, const Seen& seen, int key_bytes) {
   int rows = 0;
   const dim3 grid = idx_grid((int64_t)nb * bsz * n, nb, bsz * n, &rows);
   const bool far = (int64_t)bsz * nb * key_bytes >= 7 << 19;   // 3.5 of 4 MB
-  return t.base + rounds_of((int64_t)grid.x * grid.y) * (t.step + t.rows * min(rows, nb) / 1024.0) +
-         (far ? t.far * 1e-6 * bsz * n * nb : 0.0);
+  return t.base + rounds_of(workgroups_seen(grid.y, rows, (int)grid.x, seen)) *
+                      (t.step + t.rows * fmin((double)rows, seen.last) / 1024.0) +
+         (far ? t.far * 1e-6 * bsz * n * seen.mean : 0.0);
 }
 
 }  // namespace dsv41
@@ -1097,10 +1124,11 @@ extern "C" int dsv41_indexer_score(const void* q, const void* w_raw, float w_sca
     // keys 10.0 us with one, 10.6 with two)
     const int nq = candidates || heads > 32 || (heads == 32 && nb <= 384) ? 1 : 2;
     double time = 0.0;
-    const int rows = prefill_rows(groups, nb, nq, &time);
+    const Seen seen = seen_keys(start_pos, n, ratio, nb);
+    const int rows = prefill_rows(groups, nb, seen, nq, &time);
     const int hc = head_class(heads);
     const ChunkUs& t = kChunkBf16Masked[hc];
-    const bool gains = !candidates || t.base + t.unit * time < one_query_us(kOneQueryBf16[hc], bsz, n, nb, 2 * dim) *
+    const bool gains = !candidates || t.base + t.unit * time < one_query_us(kOneQueryBf16[hc], bsz, n, nb, seen, 2 * dim) *
                                                                    (aligned16(w_raw) ? 0.95 : kPlainOneQuery);
     const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
     const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
@@ -1199,12 +1227,13 @@ extern "C" int dsv41_indexer_score_fp8(const void* q, const void* w_raw, float w
   if (n >= 8 && (heads == 64 || heads == 32 || heads == 16)) {
     const int64_t groups = (int64_t)bsz * ((n + kPfQueries - 1) / kPfQueries);
     double time = 0.0;
-    const int rows = prefill_rows(groups, nb, !candidates && heads <= 32 ? 2 : 1, &time);
+    const Seen seen = seen_keys(start_pos, n, ratio, nb);
+    const int rows = prefill_rows(groups, nb, seen, !candidates && heads <= 32 ? 2 : 1, &time);
     const int hc = head_class(heads);
     const ChunkUs& t = candidates ? kChunkFp8Masked[hc] : kChunkFp8[hc];
     const bool staged = aligned16(w_raw) && aligned16(k_scale) && ks_bstride % 16 == 0;
     const bool gains = t.base + t.unit * time <
-                       one_query_us(kOneQueryFp8[hc], bsz, n, nb, dim) * (staged ? 0.95 : kPlainOneQuery);
+                       one_query_us(kOneQueryFp8[hc], bsz, n, nb, seen, dim) * (staged ? 0.95 : kPlainOneQuery);
     const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
     const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_PF8_CASE(HT_, NQ_, CAND_)                                                                       \
@@ -1278,8 +1307,10 @@ static int mx_score_entry(const char* what, bool kf8, const uint8_t* q_codes, co
     const int rows = mx_chunk_rows(groups, nb);
     const int hc = head_class(heads);
     const MxChunkUs& t = kChunkMx[hc];
-    const bool gains = t.base + rounds_of(groups * ((nb + rows - 1) / rows)) * (t.step + t.rows * min(rows, nb) / 1024.0) <
-                       one_query_us(kOneQueryMx[hc], bsz, n, nb, dim / 2);
+    const Seen seen = seen_keys(start_pos, n, ratio, nb);
+    const int64_t wgs = workgroups_seen(groups, rows, (nb + rows - 1) / rows, seen);
+    const bool gains = t.base + rounds_of(wgs) * (t.step + t.rows * fmin((double)rows, seen.last) / 1024.0) <
+                       one_query_us(kOneQueryMx[hc], bsz, n, nb, seen, dim / 2);
     const dim3 cgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_MXCHUNK_CASE(HT_, CAND_)                                                                        \
     if (gains && heads == HT_ * 16 && (candidates != nullptr) == CAND_) {                                     \
