@@ -44,19 +44,22 @@ def select_candidate_blocks(scores: torch.Tensor, lens, topk_blocks: int,
                                  _lens_tensor(lens, scores.device))
 
 
-# Queries per sequence from which bf16 and MXFP4 keys take the scoring and the selection as two calls:
-# the scoring kernel then reads each key once per several queries, where the fused form's reads every
-# key for every query. Only masked layers meet the choice (without a mask the fused form stops at 8
-# queries anyway). 32 heads, fused against score + select: bf16 keys 8 queries x 65,536 keys 42.9
-# against 30.1 us, 64 x 8,192 22.0 against 21.7 us, 2,048 x 32,768 1,181 against 470 us; MXFP4 keys
-# 8 x 65,536 38.0 against 27.5 us, 64 x 8,192 21.8 against 21.3 us, 2,048 x 32,768 655 against 351 us;
-# no size measured from 8 queries on favoured the fused form.
-CHUNK_QUERIES = 8
-# The same choice over fp8 keys, whose fused form wins on small chunks (fused against two calls, 9 x 8,192
-# keys, 64 heads 17.7 against 26.1 us, 64 x 2,048 17.4 against 22.7 us) and loses from half a million
-# scores on (64 x 8,192, 32 heads 26.4 against 23.4 us, 8 x 65,536 43.8 against 30.0 us, 2,048 x 32,768
-# 1,048 against 475 us).
-CHUNK_SCORES_FP8 = 1 << 19
+def _score_then_select(queries: int, nb: int, topk: int, mxfp4: bool) -> bool:
+    """Whether a chunk of 8 and more queries under a candidate mask takes scoring and selection as two calls
+    instead of the fused form. The two calls read each key once per several queries; the fused form writes no
+    scores and starts sooner. Whole Indexer.forward calls, 8 to 300 queries of 1 and 4 sequences over 2,000 to
+    65,000 keys, 32 and 64 heads, top-128 to top-1,024 (us, fused against two calls, bf16 keys, 32 heads):
+    * up to 8,192 keys two calls (4 x 32 queries x 8,032 12 % less time, at worst 1 % more);
+    * beyond, from 786,432 scores on (64 x 16,064, top-512 7 % less, 300 x 16,300 28 % less; 8 x 24,008 6 % more),
+      lists of 512 and more over 32,768 keys at once (8 x 65,008 20 % less);
+    * MXFP4 keys of 24,577 to 32,768, the longest rows one workgroup selects, with lists below 1,024 from
+      3 x 2^20 (64 x 32,764 9 % more, 200 x 32,200 26 % less)."""
+    scores = queries * nb
+    if nb <= 8192:
+        return True
+    if mxfp4 and 24576 < nb <= 32768 and topk < 1024:
+        return scores >= 3 << 20
+    return scores >= 3 << 18 or (topk >= 512 and nb > 32768)
 
 
 @functools.lru_cache(maxsize=256)
@@ -124,6 +127,11 @@ class Indexer(torch.nn.Module):
                                self.k_norm.eps)
         cache.index_k[:k_raw.shape[0], g0:g0 + k_raw.shape[1]] = staged
 
+    def _fused(self, bsz: int, n: int, nb: int, cand, mxfp4: bool = False) -> bool:
+        """Whether to ask the fused scoring and selection for this chunk."""
+        return n < 8 or (cand is not None
+                         and not _score_then_select(bsz * n, nb, self.index_topk, mxfp4))
+
     def forward(self, x: torch.Tensor, qr: torch.Tensor, start_pos: int, offset: int,
                 cos, sin, index_k: torch.Tensor, shared) -> torch.Tensor:
         """x [b,n,dim], qr [b,n,q_lora]; index_k [b, nb, Di] (the owner's cache, in place), or
@@ -144,7 +152,7 @@ class Indexer(torch.nn.Module):
                 raise ValueError("an MXFP4 index cache holds fp4 fake-quantized keys; QAT is disabled")
             q_mx = _abi.index_q_prep_mxfp4(q, cos, sin, rd, start_pos)
             nb = index_k.codes.shape[1]
-            if not self.is_candidate_source and n < CHUNK_QUERIES:
+            if not self.is_candidate_source and self._fused(bsz, n, nb, cand, mxfp4=True):
                 idx = _abi.indexer_topk_mxfp4(q_mx, w_raw, w_scale, index_k.codes, index_k.scales, nb, start_pos,
                                               self.ratio, self.index_topk, offset, cand)
                 if idx is not None:
@@ -158,7 +166,7 @@ class Indexer(torch.nn.Module):
                 _abi.index_q_prep(q, cos, sin, rd, start_pos)
             nb = index_k.codes.shape[1]
             if (not self.is_candidate_source and q.dtype == torch.bfloat16
-                    and (n < CHUNK_QUERIES or bsz * n * nb < CHUNK_SCORES_FP8)):
+                    and self._fused(bsz, n, nb, cand)):
                 idx = _abi.indexer_topk_fp8(q, w_raw, w_scale, index_k.codes, index_k.scales, index_k.rb, nb, start_pos,
                                             self.ratio, self.index_topk, offset, cand)
                 if idx is not None:
@@ -170,7 +178,8 @@ class Indexer(torch.nn.Module):
                 q = _abi.rope_tail(q, rd, cos, sin, start_pos, 1)
             else:
                 _abi.index_q_prep(q, cos, sin, rd, start_pos)
-            if not self.is_candidate_source and q.dtype == torch.bfloat16 and n < CHUNK_QUERIES:
+            if (not self.is_candidate_source and q.dtype == torch.bfloat16
+                    and self._fused(bsz, n, index_k.shape[1], cand)):
                 # decode shapes the fused form serves: the same selection, the scores never written
                 idx = _abi.indexer_topk(q, w_raw, w_scale, index_k, start_pos, self.ratio, self.index_topk, offset,
                                         cand)
