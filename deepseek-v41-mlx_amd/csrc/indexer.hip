@@ -409,7 +409,7 @@ __device__ __forceinline__ f32x4 mfma_mxfp4_tile(uint4 a, int sa, int ht, uint4 
 // fp8 keys: an fp4 e2m1 query (A, cbsz = 4) against e4m3 keys (B, blgp = 0). With 8-bit
 // operands the 16x16x128 instruction takes a lane group's 32 bytes as two 16-channel halves:
 // lane group g supplies channels [16g, 16g+16) in bytes 0-15 and [64+16g, 64+16g+16) in bytes
-// 16-31 (a one-wave probe on the box pinned this against a float64 reference), while its scale
+// 16-31 (a one-wave probe pinned this against a float64 reference), while its scale
 // byte is that of channel block g, like the fp4 operand's contiguous 32 channels. Products are
 // exact; the probe measured the instruction's sums within 3e-5 of max|D| of the exact sum (a
 // float32 channel-order sum of the same products was exact), so these scores are close to, not
@@ -575,9 +575,9 @@ __global__ __launch_bounds__(kMxThreads) void indexer_score_mx_kernel(
 // leave as one 256-byte store per query. Bound by issue: a 16 x 16 tile of one head tile is one fp4
 // MFMA and 8 VALU instructions (max and fma per product, 32 cycles). 1,999 queries x 16,359 keys,
 // causal: 32 heads 200 us with a workgroup per query (bound by its key loads and 64-byte stores) ->
-// 121 us; 64 heads 188 us, 16 heads 63 us here. NQ * HT = 8 head tiles at three waves per SIMD (168
-// registers); the same at 32 heads with 4 tiles 141 us, 16 tiles 154 us, 8 tiles in 512-thread
-// workgroups of 128 registers 127 us.
+// 121 us; 64 heads 188 us, 16 heads 63 us here. NQ * HT = 8 head tiles, 123 to 126 registers at 64 and
+// 32 heads (four waves per SIMD), 129 at 16 heads (three); the same at 32 heads with 4 tiles 141 us, 16
+// tiles 154 us, 8 tiles in 512-thread workgroups 127 us.
 template <int HT, bool CAND>
 __global__ __launch_bounds__(kMxChunkThreads, 3) void indexer_mx_chunk_kernel(
     const uint8_t* __restrict__ qcodes, const uint8_t* __restrict__ qscales, const bf16_t* __restrict__ w_raw,
@@ -700,7 +700,7 @@ __device__ __forceinline__ uint32_t nonzero_bytes(uint32_t v) {
 }
 
 // NQ queries per wave, 8 per workgroup. NQ = 1: 8 waves, 4 per SIMD (128 registers, two workgroups
-// share a CU). NQ = 2 (16 and 32 heads, no mask): 4 waves, 3 per SIMD (168 registers, three
+// share a CU). NQ = 2 (16 heads, and 32 past short bf16 caches, no mask): 4 waves, 3 per SIMD (168 registers, three
 // workgroups), each key operand read from LDS once for two queries; one per wave, the 32-head LDS
 // reads take as long as the MFMAs. 4,096 queries x 36,864 keys, 32 heads 993 -> 926 us, 2,048 x 8,192
 // 116 -> 111 us, 16 heads 78 -> 74 us. Under a mask two queries share few empty tiles: 32 heads,
@@ -709,7 +709,8 @@ __device__ __forceinline__ uint32_t nonzero_bytes(uint32_t v) {
 // F8: e4m3 keys with ue8m0 scales, dequantized once per workgroup on their way into the ring (exact
 // in bf16, indexer_decode_kernel's operands bit for bit), through registers one chunk ahead instead of
 // the LDS copies. They ran a workgroup per query on indexer_decode_kernel: 2,048 queries x 8,192 keys,
-// 32 heads 199 -> 115 us, 64 heads 280 -> 213 us; masked 2,048 x 32,768 845 -> 388 us.
+// 32 heads 199 -> 115 us, 64 heads 280 -> 213 us; masked 2,048 x 32,768 845 -> 388 us. The unmasked 64-head
+// form sits at its 128 registers and spills 6 (28 bytes of scratch per lane).
 template <int HT, int NQ, bool CAND, bool F8>
 __global__ __launch_bounds__(64 * kPfQueries / NQ, NQ == 1 ? 4 : 3) void indexer_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ w_raw, float w_scale, const void* __restrict__ kcache,
@@ -1128,12 +1129,13 @@ extern "C" int dsv41_indexer_score(const void* q, const void* w_raw, float w_sca
     const int rows = prefill_rows(groups, nb, seen, nq, &time);
     const int hc = head_class(heads);
     const ChunkUs& t = kChunkBf16Masked[hc];
-    const bool gains = !candidates || t.base + t.unit * time < one_query_us(kOneQueryBf16[hc], bsz, n, nb, seen, 2 * dim) *
-                                                                   (aligned16(w_raw) ? 0.95 : kPlainOneQuery);
+    const bool gains =
+        !candidates || t.base + t.unit * time < one_query_us(kOneQueryBf16[hc], bsz, n, nb, seen, 2 * dim) *
+                                                    (aligned16(w_raw) ? 0.95 : kPlainOneQuery);
     const int cvec = candidates && nb % 16 == 0 && aligned16(candidates) ? 1 : 0;
     const dim3 pgrid((unsigned)((nb + rows - 1) / rows), (unsigned)groups);
 #define DSV41_PF_CASE(HT_, NQ_, CAND_)                                                                      \
-    if (gains && heads == HT_ * 16 && nq == NQ_ && (candidates != nullptr) == CAND_) {                                           \
+    if (gains && heads == HT_ * 16 && nq == NQ_ && (candidates != nullptr) == CAND_) {                      \
       hipLaunchKernelGGL((indexer_prefill_kernel<HT_, NQ_, CAND_, false>), pgrid, dim3(64 * kPfQueries / NQ_), 0, \
                          stream, (const bf16_t*)q, (const bf16_t*)w_raw, w_scale, index_k, k_bstride, nullptr, \
                          0, 0, candidates, scores, n, nb, start_pos, ratio, rows, cvec);                      \

@@ -1150,9 +1150,8 @@ struct MlaPlan {
 // Many queries (prefill): one workgroup per (query, head group) over the whole list, 64 heads
 // per workgroup when there are more than 32. Few queries (decode): (query, 32-head, split)
 // workgroups, the list split in whole 32-row steps until about 256 workgroups exist -- or 512,
-// two per CU, when there are already >= 128 (query, head group) units or the list is >= 1024
-// entries long (measured: bs32 / 640 rows is fastest at 4 splits, B=16 / 1152 rows and B=64 at
-// ~2 workgroups per CU). Splits of at most kPairList entries with head_dim <= 512 run the PAIR
+// two per CU, when there are already >= 128 (query, head group) units (measured: bs32 / 640 rows
+// is fastest at 4 splits, B=16 / 1,152 rows at 256 workgroups, B=64 at ~2 workgroups per CU). Splits of at most kPairList entries with head_dim <= 512 run the PAIR
 // instance (~77 KB of LDS, a two-slot ring), the rest one ~160 KB workgroup per CU. A workgroup
 // stages at most kMaxList list entries.
 //

@@ -604,10 +604,11 @@ def linear_rows_wide(rows: int, k: int, n: int, splits: int) -> bool:
 
 @functools.lru_cache(maxsize=4096)
 def linear_rows_splits(k: int, n: int, rows: int = 64) -> int:
-    """(Of the sizes alone; kept per size, the search takes longer than the launch it plans.) Contraction ranges for dsv41_linear_rows (whole 64-channel steps, at most 64). At 33-64 rows
-    the ranges whose wide tiles (linear_rows_wide) make the most workgroups when some do; otherwise the most
-    that keep the n / 32 x ranges workgroups within one wave of the chip (256: one workgroup per
-    CU; a 320-workgroup wq_a ran a second round of 64 and took 9.0 us)."""
+    """Contraction ranges for dsv41_linear_rows (whole 64-channel steps, at most 64). At 33-64 rows the ranges
+    whose wide tiles (linear_rows_wide) make the most workgroups when some do; otherwise the most that
+    keep the n / 32 x ranges workgroups within one wave of the chip (256: one workgroup per CU; a
+    320-workgroup wq_a ran a second round of 64 and took 9.0 us). A function of the sizes alone, kept per
+    size: the search takes longer than the launch it plans."""
     wide = [((n // linear_rows_wide_tile(rows, k, n, s)) * s, s) for s in range(1, 65)
             if k % (64 * s) == 0 and linear_rows_wide(rows, k, n, s)]
     if wide:

@@ -149,7 +149,9 @@ int dsv41_compress_pool(const float* kv, const float* score, float* kv_state, fl
  * weights w0 [n0, k], w1 [n1, k]. Each weight enters the bf16 matrix cores as three bf16 numbers whose
  * sum it is exactly, so products are exact and sums float32. k a multiple of 64, n0 and n1 of 128;
  * dtype (of x) is BF16. The workspace is dsv41_linear_f32_pair_workspace_bytes(...) bytes, 16-byte
- * aligned (0: none). */
+ * aligned (0: none). The size is that of these rows and does not grow with them (few rows are cut into
+ * more ranges): a buffer for several row counts takes the largest of their sizes. A NaN or infinite
+ * result costs its tile a second pass on the matrix cores. */
 size_t dsv41_linear_f32_pair_workspace_bytes(int32_t rows, int32_t k, int32_t n0, int32_t n1);
 int dsv41_linear_f32_pair(const void* x, const float* w0, const float* w1, float* y0, float* y1,
                           void* workspace, size_t workspace_bytes, int32_t rows, int32_t k, int32_t n0,
@@ -158,7 +160,7 @@ int dsv41_linear_f32_pair(const void* x, const float* w0, const float* w1, float
 /* dsv41_linear_f32_pair and dsv41_compress_pool in one call, deepseek_v41_mlx/compressor.py:58-79, for
  * bf16 x [bsz, n, k], float32 weights w0, w1 [dim, k], dim 512 and ratio 2 or 4: the same latents and
  * state, bit for bit, without the projected rows as tensors. rows = bsz * n; the workspace is
- * dsv41_compress_chunk_workspace_bytes(...) bytes, 16-byte aligned. */
+ * dsv41_compress_chunk_workspace_bytes(...) bytes, 16-byte aligned, of these rows, as above. */
 size_t dsv41_compress_chunk_workspace_bytes(int32_t rows, int32_t k, int32_t dim);
 int dsv41_compress_chunk(const void* x, const float* w0, const float* w1, float* kv_state,
                          float* score_state, void* latents, const float* norm_w, void* workspace,

@@ -391,7 +391,7 @@ def test_cache_snapshot_restore_replays_a_decode_step(gpu, cache_format):
 
 
 # Scores of the block-scaled fp4 x fp8 MFMA against the exact scores: the instruction sums its
-# 128 exact products to a few 1e-5 of the result's magnitude (a one-wave probe on the box), so
+# 128 exact products to a few 1e-5 of the result's magnitude (a one-wave probe), so
 # the scores carry that error; the dequantizing fp8 scorer is exact.
 MXQ_FP8_TOL = 1e-4
 
